@@ -20,6 +20,7 @@
 #include "adjoint2d.hpp"
 #include "fft1d.hpp"
 #include "gfft.hpp"
+#include "gspec.hpp"
 #include "spectral3d.hpp"
 #include "step1d.hpp"
 #include "coop2d.hpp"
@@ -431,6 +432,8 @@ struct exmi_plan {
   long long n3 = 0;      // points of one field, N^D
   GfftCfg gcfg;          // runtime-size transforms: radices and lines per workgroup
   int gcode = 0;         // their knobs, encoded (autotuned at plan creation)
+  int g1 = 0;            // 1-D runtime size: whole rollouts in one launch (gspec.hip)
+  GfftCfg g1cfg;         // its radices (short chains of small butterflies)
   int gtuned = 0;        // 0: default knobs, 1: timed at plan creation, 2: from the tuning cache, 3: set
   // multi-pass adjoint: stage states, cotangents and the nonlinear VJP's
   // cotangent fields / products (allocated on first use)
@@ -861,21 +864,40 @@ static hipError_t irfft3(int N, long long I, cf* X, float* x, const Twiddles& tz
   return e;
 }
 
-// rfftn over the last D axes of I contiguous N^D fields with the
-// runtime-size transforms: r2c along the last axis, then c2c in place along
-// the others (innermost first). tw: the N-th roots of unity.
-static hipError_t rfft_gen(const GfftCfg& c, int D, long long I, const float* x, cf* X, const cf* tw,
-                           hipStream_t st) {
-  const int N = c.n;
-  const long long NZ = N / 2 + 1;
-  long long total = I * NZ;  // complex entries of all spectra
-  for (int d = 1; d < D; ++d) total *= N;
-  hipError_t e = launch_gfft(c, GFFT_R2C, x, X, total / NZ, 1, 0, 1, 1.f, tw, st);
-  long long inner = NZ;  // entries between neighbouring points of the axis
-  for (int ax = D - 2; ax >= 0 && e == hipSuccess; --ax) {
-    e = launch_gfft(c, GFFT_FWD, X, X, total / N, inner, inner * N, inner, 1.f, tw, st);
-    inner *= N;
+// The lines of axis ax (0 <= ax <= D - 2) of I spectra (N, ..., NZ).
+static GfftLines axis_lines(int D, int ax, int N, long long I) {
+  GfftLines g;
+  const int NZ = N / 2 + 1;
+  const bool outer3 = D == 3 && ax == 0;
+  g.nz = g.kkeep = NZ;
+  g.midn = outer3 ? N : 1;
+  g.pstride = outer3 ? (long long)N * NZ : NZ;
+  g.outer_stride = g.pstride * N;
+  g.nouter = D == 3 && ax == 1 ? I * N : I;
+  return g;
+}
+// The rows along the last axis of I fields of N^D points. With per > 0 the
+// physical rows of every `per` fields start gstride floats apart.
+static GfftLines row_lines(int D, int N, long long I, long long per, long long gstride) {
+  GfftLines g;
+  g.rows = D == 1 ? 1 : D == 2 ? N : (long long)N * N;
+  g.nlines = I * g.rows;
+  if (per > 0) {
+    g.rpg = per * g.rows;
+    g.gstride = gstride;
   }
+  return g;
+}
+
+// rfftn over the last D axes of I N^D fields with the runtime-size
+// transforms: r2c along the last axis, then c2c in place along the others
+// (innermost first). tw: the N-th roots of unity. Contiguous fields, or (see
+// row_lines) every `per` of them gstride floats apart.
+static hipError_t rfft_gen(const GfftCfg& c, int D, long long I, const float* x, cf* X, const cf* tw,
+                           hipStream_t st, long long per = 0, long long gstride = 0) {
+  hipError_t e = launch_gfft(c, GFFT_R2C, x, X, row_lines(D, c.n, I, per, gstride), 1.f, tw, st);
+  for (int ax = D - 2; ax >= 0 && e == hipSuccess; --ax)
+    e = launch_gfft(c, GFFT_FWD, X, X, axis_lines(D, ax, c.n, I), 1.f, tw, st);
   return e;
 }
 
@@ -884,21 +906,15 @@ static hipError_t rfft_gen(const GfftCfg& c, int D, long long I, const float* x,
 // pass reads src instead and X is only the intermediate (src is left
 // unchanged; in 1-D the c2r reads src).
 static hipError_t irfft_gen(const GfftCfg& c, int D, long long I, cf* X, float* x, const cf* tw, hipStream_t st,
-                            const cf* src = nullptr) {
-  const int N = c.n;
-  const long long NZ = N / 2 + 1;
-  const float r = 1.f / (float)N;
-  long long total = I * NZ, inner = NZ;
-  for (int d = 1; d < D; ++d) total *= N;
-  for (int d = 0; d < D - 2; ++d) inner *= N;
+                            const cf* src = nullptr, long long per = 0, long long gstride = 0) {
+  const float r = 1.f / (float)c.n;
   hipError_t e = hipSuccess;
   const cf* in = src ? src : X;
   for (int ax = 0; ax <= D - 2 && e == hipSuccess; ++ax) {
-    e = launch_gfft(c, GFFT_INV, in, X, total / N, inner, inner * N, inner, r, tw, st);
+    e = launch_gfft(c, GFFT_INV, in, X, axis_lines(D, ax, c.n, I), r, tw, st);
     in = X;
-    inner /= N;
   }
-  if (e == hipSuccess) e = launch_gfft(c, GFFT_C2R, in, x, total / NZ, 1, 0, 1, r, tw, st);
+  if (e == hipSuccess) e = launch_gfft(c, GFFT_C2R, in, x, row_lines(D, c.n, I, per, gstride), r, tw, st);
   return e;
 }
 
@@ -1023,6 +1039,15 @@ static int plan_create_md(const exmi_plan_desc* d, exmi_plan** out, bool gen) {
     return rc;
   }
   if (gen) gfft_cfg_from_code(N, gfft_default_code(), &p->gcfg);
+  if (gen && D == 1) {
+    p->g1 = g1d_fits(N, C, p->nf3, p->np3, d->order, d->lin_channels, p->ncoef) ? 1 : 0;
+    // the shortest chain of small butterflies: passes of at most 8 points, of
+    // 10 where that takes more than three (measured per step of one
+    // trajectory: N = 100 7.0 us as 4 5 5 against 8.7 as 10 10, N = 243 9.7 as
+    // 3 9 9 against 14.2 as 3 3 3 3 3)
+    gfft_cfg_from_code(N, 100000000 + 8 * 100000 + 2048, &p->g1cfg);
+    if (p->g1cfg.npass > 3) gfft_cfg_from_code(N, 100000000 + 10 * 100000 + 2048, &p->g1cfg);
+  }
   p->gcode = gen ? gfft_default_code() : 0;
   const long long rows = (long long)d->lin_batch * d->lin_channels, total = rows * p->nr;
   double* dL = nullptr;
@@ -1091,12 +1116,8 @@ static hipError_t irfft_md(const exmi_plan* p, long long I, cf* X, float* x, hip
   if (p->gen) return irfft_gen(p->gcfg, p->ndim, I, X, x, p->tw_col.tw, st);
   return irfft3(p->d.num_points, I, X, x, p->tw, p->tw_col, st);
 }
-// irfftn of the spectra X that leaves X unchanged (the intermediate in K)
-static hipError_t irfft_md_keep(const exmi_plan* p, long long I, const cf* X, cf* K, float* x, hipStream_t st) {
-  if (p->gen) return irfft_gen(p->gcfg, p->ndim, I, K, x, p->tw_col.tw, st, X);
-  return irfft3(p->d.num_points, I, K, x, p->tw, p->tw_col, st, X);
-}
-// The same for a fused 3-D size, each state (C N^3 floats) written to x +
+// irfftn of the spectra X of a fused 3-D size that leaves X unchanged (the
+// intermediate in K), each state (C N^3 floats) written to x +
 // b * xstride (a strided batch such as a trajectory buffer).
 static hipError_t irfft3_keep_strided(const exmi_plan* p, const cf* X, cf* K, float* x, long long xstride,
                                       hipStream_t st) {
@@ -1162,6 +1183,32 @@ static bool xstage_kind(const exmi_plan* p) {
 static hipError_t nonlinear3d_products(exmi_plan* p, const NL3DArgs& a, const cf* X, hipStream_t st,
                                        const cf** ph, bool no_x = false) {
   *ph = p->F3;
+  if (p->gen && p->ndim >= 2 && p->kmax >= 0 && gprod_fits(p->gcfg, a)) {
+    // the fields with the first inverse axis, the rows with the products, and
+    // the forward axes; what the dealias cutoff makes zero or the combine
+    // does not read is left out
+    const int N = p->d.num_points, NZ = N / 2 + 1;
+    const int kk = (p->kmax < NZ - 1 ? p->kmax : NZ - 1) + 1, cut = p->kmax < N ? p->kmax : N;
+    const float r = 1.f / (float)N;
+    const cf* tw = p->tw_col.tw;
+    cf* P = (cf*)p->PR3;  // allocated to hold the products as spectra
+    hipError_t e = launch_gfields(p->gcfg, a, X, p->F3, r, kk, tw, st);
+    if (e == hipSuccess && p->ndim == 3) {
+      GfftLines y = axis_lines(3, 1, N, p->ninst * p->nf3);
+      y.kkeep = kk;
+      y.pcut = cut;
+      e = launch_gfft(p->gcfg, GFFT_INV, p->F3, p->F3, y, r, tw, st);
+    }
+    if (e == hipSuccess) e = launch_gprod(p->gcfg, a, p->F3, P, r, kk, tw, st);
+    for (int ax = p->ndim - 2; ax >= 0 && e == hipSuccess; --ax) {
+      GfftLines g = axis_lines(p->ndim, ax, N, p->ninst * p->np3);
+      g.kkeep = kk;
+      g.cut = g.pcut = cut;
+      e = launch_gfft(p->gcfg, GFFT_FWD, P, P, g, 1.f, tw, st);
+    }
+    *ph = P;
+    return e;
+  }
   if (p->gen) {
     hipError_t e = launch_fields3d(a, X, p->F3, st);
     if (e == hipSuccess) e = irfft_md(p, p->ninst * p->nf3, p->F3, p->R3, st);
@@ -1284,6 +1331,40 @@ static hipError_t stages3d(exmi_plan* p, Stage3DArgs& sa, hipStream_t st, cf* em
   return e;
 }
 
+// 1-D plans of a runtime size that fit LDS (p->g1): n steps in one launch,
+// states to out + b * out_bs + t * out_ts (only the last, at out + b * out_bs,
+// with final_only); roundtrip: every step starts from the emitted float32
+// state, else the spectrum is carried.
+static int enqueue_g1d(exmi_plan* p, const float* u0, long long u0_bs, float* out, long long out_bs,
+                       long long out_ts, int n, int final_only, int roundtrip, hipStream_t st) {
+  G1dArgs g;
+  fill_nl3d(p, g.nl);
+  // alias-free quadratic products: u u_x and (1/2)(u^2)_x agree on every
+  // retained mode (the rule of the compiled 1-D sizes in exmi_plan_create)
+  if (g.nl.kind == NL_CONV_NONCONS && !(p->d.flags & EXMI_FLAG_EXACT_FORM) && g.nl.channels == 1 && p->kmax >= 0 &&
+      3LL * p->kmax < g.nl.N) {
+    g.nl.kind = NL_CONV_CONS;
+    g.nl.nf = 1;
+  }
+  g.order = p->d.order;
+  g.ncoef = p->ncoef;
+  g.lin_batch = p->d.lin_batch;
+  g.lin_channels = p->d.lin_channels;
+  g.e_im = p->cplx ? num_coefs(p->d.order) : -1;
+  g.nsteps = n;
+  g.final_only = final_only;
+  g.roundtrip = roundtrip;
+  g.tables = p->tables;
+  g.tw = p->tw_col.tw;
+  g.u0 = u0;
+  g.u0_bs = u0_bs;
+  g.out = out;
+  g.out_bs = out_bs;
+  g.out_ts = out_ts;
+  const hipError_t e = launch_g1d(p->gtuned == 3 ? p->gcfg : p->g1cfg, g, st);
+  return e == hipSuccess ? EXMI_OK : fail(EXMI_ERR_HIP, "1-D rollout launch failed: %s", hipGetErrorString(e));
+}
+
 // One multi-pass step u_in (batch stride ibs) -> u_out (obs): forward
 // transform, ETDRK stages, inverse transform; strided states pass through
 // the staging buffer.
@@ -1292,12 +1373,15 @@ static hipError_t stages3d(exmi_plan* p, Stage3DArgs& sa, hipStream_t st, cf* em
 // evaluates N(u_hat) instead of a step (exmi_nonlinear).
 static int enqueue_step3d(exmi_plan* p, const float* u_in, long long ibs, float* u_out, long long obs,
                           hipStream_t st, bool in_f = false, bool out_f = false, bool nonlin_only = false) {
-  const int B = p->d.batch;
+  if (p->g1 && !in_f && !out_f && !nonlin_only) return enqueue_g1d(p, u_in, ibs, u_out, obs, 0, 1, 1, 0, st);
+  const int B = p->d.batch, C = p->d.num_channels;
   const long long sz = (long long)p->d.num_channels * p->n3;
   const long long szs = 2LL * p->d.num_channels * p->nr;  // floats of one spectrum
   hipError_t e = hipSuccess;
   if (in_f) {
     e = copy_batch(u_in, 2 * ibs, (float*)p->W3, szs, szs, B, st);
+  } else if (p->gen) {
+    e = rfft_gen(p->gcfg, p->ndim, p->ninst, u_in, p->W3, p->tw_col.tw, st, C, ibs);
   } else {
     const float* src = u_in;
     if (ibs != sz) {
@@ -1336,6 +1420,9 @@ static int enqueue_step3d(exmi_plan* p, const float* u_in, long long ibs, float*
   }
   if (out_f) {
     if (e == hipSuccess) e = copy_batch((const float*)X, szs, u_out, 2 * obs, szs, B, st);
+  } else if (p->gen) {
+    if (e == hipSuccess)
+      e = irfft_gen(p->gcfg, p->ndim, p->ninst, X, u_out, p->tw_col.tw, st, nullptr, C, obs);
   } else {
     float* dst = obs == sz ? u_out : p->P3;
     if (e == hipSuccess) e = irfft_md(p, p->ninst, X, dst, st);
@@ -1355,12 +1442,17 @@ static int enqueue_md_carry(exmi_plan* p, const float* u0, long long u0_bs, floa
   const int B = p->d.batch;
   const long long sz = (long long)p->d.num_channels * p->n3;
   hipError_t e = hipSuccess;
-  const float* src = u0;
-  if (u0_bs != sz) {
-    e = copy_batch(u0, u0_bs, p->P3, sz, sz, B, st);
-    src = p->P3;
+  const int C = p->d.num_channels;
+  if (p->gen) {
+    e = rfft_gen(p->gcfg, p->ndim, p->ninst, u0, p->W3, p->tw_col.tw, st, C, u0_bs);
+  } else {
+    const float* src = u0;
+    if (u0_bs != sz) {
+      e = copy_batch(u0, u0_bs, p->P3, sz, sz, B, st);
+      src = p->P3;
+    }
+    if (e == hipSuccess) e = rfft_md(p, p->ninst, src, p->W3, st);
   }
-  if (e == hipSuccess) e = rfft_md(p, p->ninst, src, p->W3, st);
   cf* cur = p->W3;
   cf* nxt = p->S3;
   Stage3DArgs sa;
@@ -1400,13 +1492,8 @@ static int enqueue_md_carry(exmi_plan* p, const float* u0, long long u0_bs, floa
                               (long long)p->d.num_channels * N * N, out_bs, st);
       continue;
     }
-    if (!p->gen) {
-      if (e == hipSuccess) e = irfft3_keep_strided(p, cur, p->K3, dst, out_bs, st);
-      continue;
-    }
-    const bool direct = out_bs == sz;
-    if (e == hipSuccess) e = irfft_md_keep(p, p->ninst, cur, p->K3, direct ? dst : p->P3, st);
-    if (e == hipSuccess && !direct) e = copy_batch(p->P3, sz, dst, out_bs, sz, B, st);
+    e = p->gen ? irfft_gen(p->gcfg, p->ndim, p->ninst, p->K3, dst, p->tw_col.tw, st, cur, C, out_bs)
+               : irfft3_keep_strided(p, cur, p->K3, dst, out_bs, st);
   }
   return e == hipSuccess ? EXMI_OK
                          : fail(EXMI_ERR_HIP, "%d-D rollout launch failed: %s", p->ndim, hipGetErrorString(e));
@@ -2240,6 +2327,8 @@ static int enqueue_rollout_nt(exmi_plan* p, int nt, const float* u0, long long u
   }
   if (n == 0) return EXMI_OK;
   if (p->md) {
+    if (p->g1)
+      return enqueue_g1d(p, u0, u0_bs, traj + off * sz, tstride, sz, n, 0, !(nt == 2 && p->md_carry), st);
     if (nt == 2 && p->md_carry) return enqueue_md_carry(p, u0, u0_bs, traj + off * sz, tstride, sz, n, 0, st);
     for (int t = 0; t < n; ++t) {
       const float* in = (t == 0 && !include_init) ? u0 : traj + (long long)(t - 1 + off) * sz;
@@ -2551,7 +2640,9 @@ static int enq_repeat_cb(exmi_plan* p, const void* a, const void* b, long long s
     return e == hipSuccess ? EXMI_OK : fail(EXMI_ERR_HIP, "copy failed: %s", hipGetErrorString(e));
   }
   if (p->md) {
-    if (effective_nt(p) == 2 && p->md_carry) return enqueue_md_carry(p, u0, s, out, sz, 0, n, 1, st);
+    const bool carry = effective_nt(p) == 2 && p->md_carry;
+    if (p->g1) return enqueue_g1d(p, u0, s, out, sz, 0, n, 1, !carry, st);
+    if (carry) return enqueue_md_carry(p, u0, s, out, sz, 0, n, 1, st);
     for (int t = 0; t < n; ++t) {
       int rc = enqueue_step3d(p, t == 0 ? u0 : out, t == 0 ? s : sz, out, sz, st);
       if (rc) return rc;
@@ -2895,7 +2986,7 @@ static int gen_transform(bool inverse, int D, int N, int count, const float* in,
   if (!inverse) {
     e = rfft_gen(c, D, count, in, (cf*)out, tw.tw, st);
   } else if (D == 1) {
-    e = launch_gfft(c, GFFT_C2R, in, out, count, 1, 0, 1, 1.f / (float)N, tw.tw, st);
+    e = launch_gfft(c, GFFT_C2R, in, out, row_lines(1, N, count, 0, 0), 1.f / (float)N, tw.tw, st);
   } else {
     size_t nr = (size_t)(N / 2 + 1);
     for (int d = 1; d < D; ++d) nr *= (size_t)N;

@@ -3,235 +3,209 @@
 // The fused step kernels are compiled per transform size (powers of two and
 // the two small mixed-radix sizes 48 and 50). Every other grid size the
 // reference accepts (_spectral.py:614-721 takes any N: odd N, 100, 513, ...)
-// runs through the kernel below: a workgroup stages `lpb` lines in LDS and
-// runs the self-sorting Stockham passes of a factorisation n = R_1 ... R_m
-// (Govindaraju et al., "High performance discrete Fourier transforms on
-// graphics processors", SC 2008): in the pass of radix R after passes whose
-// radices multiply to Ns, butterfly j reads x[j + s n/R] (s < R), multiplies
-// input s by exp(-2 pi i s (j mod Ns) / (Ns R)), forms the R-point DFT and
-// writes output q to ((j / Ns) Ns R + j mod Ns + q Ns). Each output is
-// computed directly as one R-term sum whose twiddle exponent
-// s ((j mod Ns) n/(Ns R) + q n/R) mod n indexes one table of the n-th roots
-// of unity (formed in double precision, rounded once), in LDS when it fits.
-// Radices up to 16 (and 17, 19) run as register butterflies: a thread reads
-// a butterfly's R inputs once, twiddles them and forms the R-point DFT with
-// the R-th roots from the same table; any other radix (a prime factor above
-// the largest pass) is a direct-sum pass, so every n factors.
+// runs through the passes below: a workgroup stages `lpb` lines side by side
+// in LDS and runs the self-sorting Stockham passes of a factorisation
+// n = R_1 ... R_m (Govindaraju et al., "High performance discrete Fourier
+// transforms on graphics processors", SC 2008; gfft.hpp). The twiddles index
+// one table of the n-th roots of unity (formed in double precision, rounded
+// once), in LDS when it fits. Radices up to 16 (and 17, 19) are register
+// butterflies; any other radix (a prime factor above the largest pass) is a
+// direct-sum pass, so every n factors.
+//
+// What bounds it: LDS traffic and instruction issue, not memory (four fields
+// of eight 513^2 grids along y: 90 MB in and out). Real lines run two per
+// complex transform where they are neighbouring rows of one field; divisions
+// by runtime sizes are float multiplications; the lines of a workgroup share
+// their twiddle reads and lie side by side at an odd pitch.
+// Measured (eight 513^2 fields, one transform along one axis): forward lines
+// 22 us, inverse lines 19 us, r2c 20 us, c2r 15 us, against 33, 33, 42 and
+// 43 us with one real line per transform, R^2 complex products per radix-R
+// butterfly and integer divisions; a prime pass of 199 points (N = 597, one
+// step of 100 trajectories) 60 us per step against 185 us with direct sums.
 #include <cstdio>
+#include <vector>
 
 #include "gfft.hpp"
 
 namespace exmi {
 
-constexpr int GFFT_WG = 256;
-
 struct GfftArgs {
-  GfftCfg c;
+  GfftDev d;
+  int lpb;
+  GfftLines g;
+  long long nrun;  // lines (C2C), or complex lines of one or two real lines
   const void* in;
   void* out;
-  long long nlines, inner, outer_stride, pstride;
   float scale;
   const cf* tw;
-  int tw_lds;  // 1: the twiddle table is staged in LDS (it fits beside the two line buffers)
 };
 
-// x * w, or x * conj(w) for the inverse
-template <bool INV>
-__device__ __forceinline__ cf twmul(cf x, cf w) {
-  return INV ? cf{fmaf(x.re, w.re, x.im * w.im), fmaf(x.im, w.re, -x.re * w.im)}
-             : cf{fmaf(x.re, w.re, -x.im * w.im), fmaf(x.im, w.re, x.re * w.im)};
-}
-
-// One Stockham pass of radix R (compile time) over lpb lines of n points:
-// each thread owns whole butterflies, reads its R inputs once, twiddles them,
-// forms the R-point DFT in registers (the R-th roots of unity are the table
-// entries k n / R) and writes its R outputs.
-template <int R, bool INV>
-__device__ __forceinline__ void gfft_pass_r(const cf* A, cf* B, const cf* T, int n, int Ns, int lpb, int tid) {
-  const int m = n / R;           // butterflies per line
-  const int tws = n / (Ns * R);  // twiddle stride of this pass
-  cf wr[R];
-#pragma unroll
-  for (int k = 0; k < R; ++k) wr[k] = T[k * m];
-  for (int idx = tid; idx < lpb * m; idx += GFFT_WG) {
-    const int ll = idx / m, j = idx - ll * m;
-    const int jm = j % Ns;
-    const cf* src = A + ll * n + j;
-    cf x[R];
-    x[0] = src[0];
-    const int e1 = jm * tws;  // s * e1 < n for s < R
-#pragma unroll
-    for (int s = 1; s < R; ++s) x[s] = twmul<INV>(src[s * m], T[s * e1]);
-    cf* dst = B + ll * n + (j - jm) * R + jm;
-#pragma unroll
-    for (int q = 0; q < R; ++q) {
-      cf acc = x[0];
-#pragma unroll
-      for (int s = 1; s < R; ++s) {
-        const cf w = wr[(q * s) % R];
-        const cf t = twmul<INV>(x[s], w);
-        acc.re += t.re;
-        acc.im += t.im;
-      }
-      dst[q * Ns] = acc;
-    }
-  }
-}
-
-// Any radix: each output one R-term sum whose twiddle exponents
-// s ((j mod Ns) n/(Ns R) + q n/R) mod n index the table.
-template <bool INV>
-__device__ __forceinline__ void gfft_pass_direct(const cf* A, cf* B, const cf* T, int n, int R, int Ns, int lpb,
-                                                 int tid) {
-  const int m = n / R;
-  const int tws = n / (Ns * R);
-  for (int idx = tid; idx < lpb * n; idx += GFFT_WG) {
-    const int ll = idx / n, rem = idx - ll * n;
-    const int q = rem / m, j = rem - q * m;
-    const int jm = j % Ns;
-    int es = jm * tws + q * m;
-    if (es >= n) es -= n;
-    const cf* src = A + ll * n + j;
-    cf acc = src[0];
-    int e = es;
-    for (int s = 1; s < R; ++s) {
-      const cf t = twmul<INV>(src[s * m], T[e]);
-      acc.re += t.re;
-      acc.im += t.im;
-      e += es;
-      if (e >= n) e -= n;
-    }
-    B[ll * n + (j - jm) * R + jm + q * Ns] = acc;
-  }
-}
-
-// RMAX: the largest radix run as register butterflies (8 keeps the
-// kernel's registers, and so its occupancy, low; 19 adds 9..17 and 19 for
-// plans that have such a pass).
-template <int MODE, int RMAX>
+template <int MODE, int RMAX, bool TWL>
 __global__ void __launch_bounds__(GFFT_WG) gfft_kernel(GfftArgs a) {
   extern __shared__ cf gfft_smem[];
-  const int n = a.c.n, lpb = a.c.lpb, tot = n * lpb, nz = n / 2 + 1;
-  cf* A = gfft_smem;
-  cf* B = gfft_smem + tot;
-  const int tid = threadIdx.x;
-  const long long line0 = (long long)blockIdx.x * lpb;
+  __shared__ long long b0[GFFT_MAX_LINES], b1[GFFT_MAX_LINES];
   constexpr bool INV = MODE == GFFT_INV || MODE == GFFT_C2R;
-  const cf* T = a.tw;
-  if (a.tw_lds) {
-    cf* Tl = gfft_smem + 2 * tot;
-    for (int i = tid; i < n; i += GFFT_WG) Tl[i] = a.tw[i];
-    T = Tl;
-  }
-  // load: consecutive threads read consecutive addresses (along the line for
-  // contiguous lines, across neighbouring lines for a strided axis)
-  const bool along = MODE != GFFT_FWD && MODE != GFFT_INV ? true : a.pstride == 1;
-  for (int idx = tid; idx < tot; idx += GFFT_WG) {
-    const int ll = along ? idx / n : idx % lpb;
-    const int pt = along ? idx - ll * n : idx / lpb;
-    const long long gl = line0 + ll;
-    cf v = cf{0.f, 0.f};
-    if (gl < a.nlines) {
-      if constexpr (MODE == GFFT_R2C) {
-        v = cf{static_cast<const float*>(a.in)[gl * n + pt], 0.f};
-      } else if constexpr (MODE == GFFT_C2R) {
-        const bool upper = pt > n / 2;
-        const int k = upper ? n - pt : pt;
-        v = static_cast<const cf*>(a.in)[gl * nz + k];
-        if (k == 0 || 2 * k == n) v.im = 0.f;
-        if (upper) v.im = -v.im;
-      } else {
-        const long long base = (gl / a.inner) * a.outer_stride + gl % a.inner;
-        v = static_cast<const cf*>(a.in)[base + (long long)pt * a.pstride];
-      }
+  constexpr bool REAL = MODE == GFFT_R2C || MODE == GFFT_C2R;
+  const int n = a.d.n, nz = n / 2 + 1, tid = threadIdx.x;
+  const long long run0 = (long long)blockIdx.x * a.lpb;
+  const int L = (int)(a.nrun - run0 < a.lpb ? a.nrun - run0 : a.lpb);
+  const int pitch = gfft_pitch(a.lpb);
+  cf* A = gfft_smem;
+  cf* B = gfft_smem + n * pitch;
+  // TWL: the twiddle table is staged in LDS (it fits beside the two line buffers)
+  const cf* T = TWL ? gfft_smem + 2 * n * pitch : a.tw;
+  if constexpr (TWL)
+    for (int i = tid; i < n; i += GFFT_WG) gfft_smem[2 * n * pitch + i] = a.tw[i];
+  // where each line starts: C2C b0; real lines: the row numbers (b1 < 0: one row)
+  if (tid < L) {
+    const long long run = run0 + tid;
+    if constexpr (REAL) {
+      const long long per = (a.g.rows + 1) / 2, f = run / per, q = run - f * per;
+      b0[tid] = f * a.g.rows + 2 * q;
+      b1[tid] = 2 * q + 1 < a.g.rows ? b0[tid] + 1 : -1;
+    } else {
+      const int mk = gfft_midkeep(a.g.midn, a.g.cut);
+      const long long r = run / a.g.kkeep, o = r / mk;
+      b0[tid] = o * a.g.outer_stride + (long long)gfft_kept((int)(r - o * mk), mk, a.g.midn) * a.g.nz + run % a.g.kkeep;
     }
-    A[ll * n + pt] = v;
   }
   __syncthreads();
-  int Ns = 1;
-  for (int p = 0; p < a.c.npass; ++p) {
-    const int R = a.c.radix[p];
-    switch (R) {
-#define EXMI_GFFT_R(RR)                                          \
-  case RR:                                                       \
-    if constexpr (RR <= RMAX) {                                  \
-      gfft_pass_r<RR, INV>(A, B, T, n, Ns, lpb, tid);            \
-    } else {                                                     \
-      gfft_pass_direct<INV>(A, B, T, n, R, Ns, lpb, tid);        \
-    }                                                            \
-    break;
-      EXMI_GFFT_R(2) EXMI_GFFT_R(3) EXMI_GFFT_R(4) EXMI_GFFT_R(5) EXMI_GFFT_R(6) EXMI_GFFT_R(7)
-      EXMI_GFFT_R(8) EXMI_GFFT_R(9) EXMI_GFFT_R(10) EXMI_GFFT_R(11) EXMI_GFFT_R(12) EXMI_GFFT_R(13)
-      EXMI_GFFT_R(14) EXMI_GFFT_R(15) EXMI_GFFT_R(16) EXMI_GFFT_R(17) EXMI_GFFT_R(19)
-#undef EXMI_GFFT_R
-      default: gfft_pass_direct<INV>(A, B, T, n, R, Ns, lpb, tid); break;
+  const float rL = 1.f / (float)L, rn = a.d.rn, rnz = 1.f / (float)nz;
+  auto real_at = [&](long long row) {
+    return a.g.rpg > 0 ? (row / a.g.rpg) * a.g.gstride + (row % a.g.rpg) * n : row * n;
+  };
+  // load: consecutive threads read consecutive addresses (along the line for
+  // contiguous lines, across neighbouring lines for a strided axis)
+  if constexpr (MODE == GFFT_R2C) {
+    const float* in = static_cast<const float*>(a.in);
+    for (int idx = tid; idx < L * n; idx += GFFT_WG) {
+      const int ll = fdiv(idx, rn), pt = idx - ll * n;
+      cf v = cf{in[real_at(b0[ll]) + pt], 0.f};
+      if (b1[ll] >= 0) v.im = in[real_at(b1[ll]) + pt];
+      A[pt * pitch + ll] = v;
     }
-    __syncthreads();
-    cf* t = A;
-    A = B;
-    B = t;
-    Ns *= R;
+  } else if constexpr (MODE == GFFT_C2R) {
+    const cf* in = static_cast<const cf*>(a.in);
+    for (int idx = tid; idx < L * nz; idx += GFFT_WG) {
+      const int ll = fdiv(idx, rnz), k = idx - ll * nz;
+      cf p = in[b0[ll] * nz + k], q = b1[ll] >= 0 ? in[b1[ll] * nz + k] : cf{0.f, 0.f};
+      const bool self = k == 0 || 2 * k == n;
+      if (self) p.im = q.im = 0.f;
+      A[k * pitch + ll] = cf{p.re - q.im, p.im + q.re};
+      if (!self) A[(n - k) * pitch + ll] = cf{p.re + q.im, q.re - p.im};
+    }
+  } else {
+    const cf* in = static_cast<const cf*>(a.in);
+    for (int idx = tid; idx < L * n; idx += GFFT_WG) {
+      const int pt = fdiv(idx, rL), ll = idx - pt * L;
+      const bool zero = INV && a.g.pcut >= 0 && pt > a.g.pcut && n - pt > a.g.pcut;
+      A[pt * pitch + ll] = zero ? cf{0.f, 0.f} : in[b0[ll] + pt * a.g.pstride];
+    }
   }
+  __syncthreads();
+  const cf* Z = gfft_run<INV, RMAX>(A, B, T, a.d, L, pitch, tid, GFFT_WG);
   // store
-  const int nout = MODE == GFFT_R2C ? nz : n;
-  for (int idx = tid; idx < lpb * nout; idx += GFFT_WG) {
-    const int ll = along ? idx / nout : idx % lpb;
-    const int pt = along ? idx - ll * nout : idx / lpb;
-    const long long gl = line0 + ll;
-    if (gl >= a.nlines) continue;
-    const cf v = A[ll * n + pt];
-    if constexpr (MODE == GFFT_R2C) {
-      static_cast<cf*>(a.out)[gl * nz + pt] = v;
-    } else if constexpr (MODE == GFFT_C2R) {
-      static_cast<float*>(a.out)[gl * n + pt] = a.scale * v.re;
-    } else {
-      const long long base = (gl / a.inner) * a.outer_stride + gl % a.inner;
-      static_cast<cf*>(a.out)[base + (long long)pt * a.pstride] = a.scale * v;
+  if constexpr (MODE == GFFT_R2C) {
+    cf* out = static_cast<cf*>(a.out);
+    for (int idx = tid; idx < L * nz; idx += GFFT_WG) {
+      const int ll = fdiv(idx, rnz), k = idx - ll * nz;
+      const cf zk = Z[k * pitch + ll];
+      if (b1[ll] < 0) {
+        out[b0[ll] * nz + k] = zk;
+      } else {
+        cf p, q;
+        unpack_pair(zk, Z[(k == 0 ? 0 : n - k) * pitch + ll], p, q);
+        out[b0[ll] * nz + k] = p;
+        out[b1[ll] * nz + k] = q;
+      }
+    }
+  } else if constexpr (MODE == GFFT_C2R) {
+    float* out = static_cast<float*>(a.out);
+    for (int idx = tid; idx < L * n; idx += GFFT_WG) {
+      const int ll = fdiv(idx, rn), pt = idx - ll * n;
+      const cf v = Z[pt * pitch + ll];
+      out[real_at(b0[ll]) + pt] = a.scale * v.re;
+      if (b1[ll] >= 0) out[real_at(b1[ll]) + pt] = a.scale * v.im;
+    }
+  } else {
+    cf* out = static_cast<cf*>(a.out);
+    for (int idx = tid; idx < L * n; idx += GFFT_WG) {
+      const int pt = fdiv(idx, rL), ll = idx - pt * L;
+      if (!INV && a.g.pcut >= 0 && pt > a.g.pcut && n - pt > a.g.pcut) continue;
+      out[b0[ll] + pt * a.g.pstride] = a.scale * Z[pt * pitch + ll];
     }
   }
 }
 
-static int smallest_factor(int n) {
-  for (int f = 2; f * f <= n; ++f)
-    if (n % f == 0) return f;
-  return n;
+GfftDev gfft_dev(const GfftCfg& c, bool reversed) {
+  GfftDev d;
+  d.n = c.n;
+  d.npass = c.npass;
+  d.rn = 1.f / (float)c.n;
+  int Ns = 1;
+  for (int i = 0; i < c.npass; ++i) {
+    GfftPass& p = d.p[i];
+    p.R = c.radix[reversed ? c.npass - 1 - i : i];
+    p.Ns = Ns;
+    p.m = c.n / p.R;
+    p.tws = c.n / (Ns * p.R);
+    p.rNs = 1.f / (float)Ns;
+    Ns *= p.R;
+  }
+  return d;
+}
+
+bool gfft_big(const GfftCfg& c) {
+  bool big = false;  // a pass of radix 9..17 or 19 to run as register butterflies
+  for (int i = 0; i < c.npass; ++i) big = big || (c.radix[i] > 8 && (c.radix[i] <= 17 || c.radix[i] == 19));
+  return big && c.reg19;
 }
 
 bool gfft_make_cfg(int n, int max_radix, int points_per_wg, GfftCfg* cfg) {
   if (n < 2 || n > GFFT_MAX_N || max_radix < 2) return false;
+  // best[d] over the divisors d of n: fewest passes, then the smallest sum of
+  // radices; the last radix of the best factorisation of d
+  std::vector<int> passes(n + 1, 1 << 20), sum(n + 1, 1 << 20), last(n + 1, 0);
+  passes[1] = sum[1] = 0;
+  for (int d = 2; d <= n; ++d) {
+    if (n % d) continue;
+    for (int r = 2; r <= d; ++r) {
+      if (d % r || passes[d / r] >= (1 << 20)) continue;
+      bool prime = true;
+      for (int f = 2; f * f <= r && prime; ++f) prime = r % f != 0;
+      if (r > max_radix && !prime) continue;
+      const int np = passes[d / r] + 1, ns = sum[d / r] + r;
+      if (np < passes[d] || (np == passes[d] && ns < sum[d])) {
+        passes[d] = np;
+        sum[d] = ns;
+        last[d] = r;
+      }
+    }
+  }
+  if (passes[n] > GFFT_MAX_PASS) return false;
   GfftCfg c;
   c.n = n;
-  // prime factors in ascending order, merged greedily into passes of at most
-  // max_radix points (a larger prime is a pass of its own)
-  int rest = n, acc = 1;
-  while (rest > 1) {
-    const int f = smallest_factor(rest);
-    rest /= f;
-    if (acc > 1 && acc * f > max_radix) {
-      if (c.npass >= GFFT_MAX_PASS) return false;
-      c.radix[c.npass++] = acc;
-      acc = 1;
-    }
-    acc *= f;
-  }
-  if (acc > 1) {
-    if (c.npass >= GFFT_MAX_PASS) return false;
-    c.radix[c.npass++] = acc;
-  }
+  // the radices without a register butterfly first (see gfft_pass_direct)
+  for (int big = 1; big >= 0; --big)
+    for (int d = n; d > 1; d /= last[d])
+      if ((last[d] > 19) == (big == 1)) c.radix[c.npass++] = last[d];
   const int lpb = points_per_wg / n;
-  c.lpb = lpb < 1 ? 1 : lpb;
-  if (c.lpb * n > GFFT_MAX_N) c.lpb = 1;  // two line buffers stay within 64 KiB of LDS
+  c.lpb = lpb < 1 ? 1 : lpb > GFFT_MAX_LINES ? GFFT_MAX_LINES : lpb;
+  // two line buffers stay within 64 KiB of LDS (less the line starts)
+  while (c.lpb > 1 && sizeof(cf) * 2 * n * gfft_pitch(c.lpb) > GFFT_LDS_MAX - 2048) --c.lpb;
   *cfg = c;
   return true;
 }
 
-static const int k_gfft_cands[] = {4 * 100000 + 1024,  8 * 100000 + 1024,  16 * 100000 + 1024,
-                                   4 * 100000 + 2048,  8 * 100000 + 2048,  16 * 100000 + 2048,
-                                   8 * 100000 + 512,   8 * 100000 + 4096,  100000000 + 16 * 100000 + 1024,
-                                   100000000 + 16 * 100000 + 2048, 100000000 + 8 * 100000 + 2048};
+static const int k_gfft_cands[] = {8 * 100000 + 512,   8 * 100000 + 1024,
+                                   8 * 100000 + 2048,  8 * 100000 + 4096,
+                                   100000000 + 10 * 100000 + 1024, 100000000 + 10 * 100000 + 2048,
+                                   100000000 + 16 * 100000 + 512,  100000000 + 16 * 100000 + 1024,
+                                   100000000 + 16 * 100000 + 2048, 100000000 + 16 * 100000 + 4096,
+                                   100000000 + 8 * 100000 + 1024,  100000000 + 8 * 100000 + 2048};
 int gfft_num_candidates() { return (int)(sizeof k_gfft_cands / sizeof k_gfft_cands[0]); }
 int gfft_candidate(int i) { return k_gfft_cands[i]; }
-int gfft_default_code() { return 8 * 100000 + 2048; }
+int gfft_default_code() { return 100000000 + 8 * 100000 + 2048; }
 bool gfft_cfg_from_code(int n, int code, GfftCfg* cfg) {
   const int flag = code / 100000000, max_radix = (code / 100000) % 1000;
   if (code <= 100000 || flag > 1 || !gfft_make_cfg(n, max_radix, code % 100000, cfg)) return false;
@@ -239,34 +213,37 @@ bool gfft_cfg_from_code(int n, int code, GfftCfg* cfg) {
   return true;
 }
 
-hipError_t launch_gfft(const GfftCfg& c, int mode, const void* in, void* out, long long nlines, long long inner,
-                       long long outer_stride, long long pstride, float scale, const cf* tw, hipStream_t st) {
-  if (nlines <= 0) return hipSuccess;
-  if (c.n < 2 || c.n > GFFT_MAX_N || c.lpb < 1 || inner < 1) return hipErrorInvalidValue;
+hipError_t launch_gfft(const GfftCfg& c, int mode, const void* in, void* out, const GfftLines& g, float scale,
+                       const cf* tw, hipStream_t st) {
+  const bool real = mode == GFFT_R2C || mode == GFFT_C2R;
+  if ((real ? g.nlines : g.nouter) <= 0) return hipSuccess;
+  if (c.n < 2 || c.n > GFFT_MAX_N || c.lpb < 1 || c.lpb > GFFT_MAX_LINES) return hipErrorInvalidValue;
   GfftArgs a;
-  a.c = c;
+  a.d = gfft_dev(c);
+  a.lpb = c.lpb;
+  a.g = g;
   a.in = in;
   a.out = out;
-  a.nlines = nlines;
-  a.inner = inner;
-  a.outer_stride = outer_stride;
-  a.pstride = pstride;
   a.scale = scale;
   a.tw = tw;
-  const long long grid = (nlines + c.lpb - 1) / c.lpb;
+  if (real) {
+    if (g.rows < 1 || g.nlines % g.rows) return hipErrorInvalidValue;
+    a.nrun = g.nlines / g.rows * ((g.rows + 1) / 2);
+  } else {
+    if (g.kkeep < 1 || g.kkeep > g.nz || g.midn < 1) return hipErrorInvalidValue;
+    a.nrun = g.nouter * gfft_midkeep(g.midn, g.cut) * g.kkeep;
+  }
+  const long long grid = (a.nrun + c.lpb - 1) / c.lpb;
   if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
-  if ((long long)c.lpb * c.n > GFFT_MAX_N && c.lpb > 1) return hipErrorInvalidValue;
-  size_t lds = sizeof(cf) * (size_t)(2 * c.lpb * c.n + c.n);
-  a.tw_lds = lds <= 65536;
-  if (!a.tw_lds) lds = sizeof(cf) * (size_t)(2 * c.lpb * c.n);
-  bool big = false;  // a pass of radix 9..17 or 19 to run as register butterflies
-  for (int i = 0; i < c.npass; ++i) big = big || (c.radix[i] > 8 && (c.radix[i] <= 17 || c.radix[i] == 19));
-  big = big && c.reg19;
-#define EXMI_GFFT_LAUNCH(MODE_)                                                                                 \
-  if (big)                                                                                                      \
-    hipLaunchKernelGGL((gfft_kernel<MODE_, 19>), dim3((unsigned)grid), dim3(GFFT_WG), lds, st, a);             \
-  else                                                                                                          \
-    hipLaunchKernelGGL((gfft_kernel<MODE_, 8>), dim3((unsigned)grid), dim3(GFFT_WG), lds, st, a);
+  const size_t buf = sizeof(cf) * 2 * (size_t)c.n * gfft_pitch(c.lpb), fixed = 2 * sizeof(long long) * GFFT_MAX_LINES;
+  size_t lds = buf + sizeof(cf) * (size_t)c.n;
+  const bool twl = lds + fixed <= GFFT_LDS_MAX;
+  if (!twl) lds = buf;
+  const bool big = gfft_big(c);
+#define EXMI_GFFT_LAUNCH(M)                                                                     \
+  hipLaunchKernelGGL((big ? (twl ? gfft_kernel<M, 19, true> : gfft_kernel<M, 19, false>)        \
+                          : (twl ? gfft_kernel<M, 8, true> : gfft_kernel<M, 8, false>)),        \
+                     dim3((unsigned)grid), dim3(GFFT_WG), lds, st, a);
   switch (mode) {
     case GFFT_FWD: EXMI_GFFT_LAUNCH(GFFT_FWD) break;
     case GFFT_INV: EXMI_GFFT_LAUNCH(GFFT_INV) break;

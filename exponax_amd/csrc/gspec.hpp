@@ -1,0 +1,39 @@
+// Launch interface of the fused passes of the runtime-size plans (gspec.hip).
+#pragma once
+#include "gfft.hpp"
+#include "spectral3d.hpp"
+
+namespace exmi {
+
+// The fields of every instance with their first inverse pass (the lines of
+// the outermost axis, 2-D and 3-D): S -> F, planes kz < kkeep and, in 3-D,
+// rows |ky| <= a.kmax only.
+hipError_t launch_gfields(const GfftCfg& c, const NL3DArgs& a, const cf* S, cf* F, float scale, int kkeep,
+                          const cf* tw, hipStream_t st);
+
+// The rows along the last axis (2-D and 3-D): every field's c2r (times
+// scale), the pointwise products, and the products' r2c: F -> P, of which
+// kz < kkeep is read and stored. gprod_fits: whether one pair of rows of all
+// fields of a trajectory fits LDS.
+bool gprod_fits(const GfftCfg& c, const NL3DArgs& a);
+hipError_t launch_gprod(const GfftCfg& c, const NL3DArgs& a, const cf* F, cf* P, float scale, int kkeep,
+                        const cf* tw, hipStream_t st);
+
+// 1-D: `nsteps` whole ETDRK steps (orders 0-4) of every trajectory in one launch.
+struct G1dArgs {
+  NL3DArgs nl;
+  GfftDev d, df;  // the inverse's passes (and the forward's); df the same in reverse order
+  int order, ncoef, lin_batch, lin_channels, e_im;
+  int nsteps, final_only;
+  int roundtrip;  // 1: every step transforms the emitted state forward again, 0: the spectrum is carried
+  const float* tables;
+  const cf* tw;
+  const float* u0;
+  long long u0_bs;
+  float* out;  // state of trajectory b after step t at out + b * out_bs + t * out_ts (final_only: the last one at out + b * out_bs)
+  long long out_bs, out_ts;
+};
+bool g1d_fits(int N, int channels, int nf, int np, int order, int lin_channels, int ncoef);
+hipError_t launch_g1d(const GfftCfg& c, G1dArgs a, hipStream_t st);
+
+}  // namespace exmi

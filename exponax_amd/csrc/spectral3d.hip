@@ -12,6 +12,7 @@
 
 #include "exmi_internal.hpp"
 #include "fft1d.hpp"
+#include "nl3d.hpp"
 #include "spectral3d.hpp"
 
 namespace exmi {
@@ -154,71 +155,6 @@ hipError_t launch_etdrk0_spec(cf* X, long long ninst, long long nr, int channels
 // Cahn-Hilliard), gradient norm (_gradient_norm.py), the three-channel
 // convections (_convection.py:104-171), the general form
 // (_general_nonlinear.py) and the coupled reactions.
-struct Mode3D {
-  float kx, ky, kz;  // kappa = (2 pi / L) k along the three axes (0 on absent ones)
-  bool keep;         // |k| <= kmax on every axis
-  bool zero;         // the mean mode
-  bool inj;          // the Kolmogorov forcing mode
-};
-
-// Signed wavenumber of index i on a full (fftfreq) axis of n points: i for
-// i <= (n - 1) / 2, else i - n (even n: the Nyquist index n/2 is -n/2).
-__device__ __forceinline__ int signed_k(int i, int n) { return i <= (n - 1) / 2 ? i : i - n; }
-
-__device__ __forceinline__ Mode3D mode3d_at(const NL3DArgs& a, int ix, int iy, int iz) {
-  const int kx = signed_k(ix, a.nx), ky = signed_k(iy, a.ny);
-  Mode3D m;
-  m.kx = a.kscale * (float)kx;
-  m.ky = a.kscale * (float)ky;
-  m.kz = a.kscale * (float)iz;
-  m.keep = (kx < 0 ? -kx : kx) <= a.kmax && (ky < 0 ? -ky : ky) <= a.kmax && iz <= a.kmax;
-  m.zero = kx == 0 && ky == 0 && iz == 0;
-  m.inj = a.inj_axis == 2 ? (kx == 0 && ky == 0 && iz == a.inj_mode) : (kx == 0 && ky == a.inj_mode && iz == 0);
-  return m;
-}
-
-__device__ __forceinline__ Mode3D mode3d(const NL3DArgs& a, long long k) {
-  const int iz = (int)(k % a.NZ);
-  const long long r = k / a.NZ;
-  return mode3d_at(a, (int)(r / a.ny), (int)(r % a.ny), iz);
-}
-
-// kappa of spatial derivative d (axis 3 - D + d)
-__device__ __forceinline__ float kap_d(const NL3DArgs& a, const Mode3D& m, int d) {
-  const int axis = 3 - a.dims + d;
-  return axis == 0 ? m.kx : axis == 1 ? m.ky : m.kz;
-}
-
-__device__ __forceinline__ cf imul(float kap, cf w) { return cf{-kap * w.im, kap * w.re}; }
-
-// Field f of instance inst at entry k (mode m) of the spectra S.
-__device__ __forceinline__ cf field_at(const NL3DArgs& a, const cf* __restrict__ S, long long inst, int f,
-                                       long long k, const Mode3D& m) {
-  if (!m.keep) return cf{0.f, 0.f};
-  if (a.kind == NL_PROJ3D && f == 1) {
-    // the curl component omega_c = (i kappa x u_hat)_c of the dealiased
-    // spectra (_projected_convection.py:8-16, 120-123); field 0 is u_c
-    const long long b = (inst - inst % a.channels) * a.Nr + k;
-    const int c = (int)(inst % a.channels);
-    const cf w0 = S[b], w1 = S[b + a.Nr], w2 = S[b + 2 * a.Nr];
-    return c == 0 ? imul(m.ky, w2) - imul(m.kz, w1) : c == 1 ? imul(m.kz, w0) - imul(m.kx, w2)
-                                                           : imul(m.kx, w1) - imul(m.ky, w0);
-  }
-  const cf w = S[inst * a.Nr + k];
-  if (a.kind == NL_GRADNORM) return imul(kap_d(a, m, f), w);
-  if (a.kind == NL_CONV_NONCONS || a.kind == NL_GENERAL) return f == 0 ? w : imul(kap_d(a, m, f - 1), w);
-  if (a.kind == NL_VORT) {
-    // 2-D (_vorticity_convection.py:78-99): psi = Laplace^-1 omega (1 at
-    // the mean mode), u = d_y psi, v = -d_x psi, omega_x, omega_y; x is
-    // axis 1, y the last axis
-    const float kx = m.ky, ky = m.kz;
-    const float lap = -(kx * kx + ky * ky);
-    const cf psi = (lap == 0.f ? 1.f : 1.f / lap) * w;
-    return f == 0 ? imul(ky, psi) : f == 1 ? imul(kx, w) : f == 2 ? imul(-kx, psi) : imul(ky, w);
-  }
-  return w;
-}
-
 __global__ void fields3d_kernel(NL3DArgs a, const cf* __restrict__ S, cf* __restrict__ F) {
   const long long total = a.ninst * a.Nr;
   for (long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x; idx < total;
@@ -347,52 +283,6 @@ __global__ void products3d_kernel(NL3DArgs a, const float* __restrict__ R, float
       }
       default: out[0] = 0.f;
     }
-  }
-}
-
-// N_hat at entry idx (instance idx / Nr) from the product spectra PH.
-__device__ __forceinline__ cf combine_at(const NL3DArgs& a, const cf* __restrict__ PH, long long idx) {
-  {
-    const long long inst = idx / a.Nr, k = idx % a.Nr;
-    const Mode3D m = mode3d(a, k);
-    const cf* ph = PH + inst * a.np * a.Nr + k;
-    cf r = cf{0.f, 0.f};
-    switch (a.kind) {
-      case NL_POLY:
-        r = a.poly_lap ? (a.scale * -(m.kx * m.kx + m.ky * m.ky + m.kz * m.kz)) * ph[0] : ph[0];
-        break;
-      case NL_GRADNORM: r = (a.zero_mode_fix && m.zero) ? cf{0.f, 0.f} : (-0.5f * a.scale) * ph[0]; break;
-      case NL_CONV_CONS: {
-        cf acc = cf{0.f, 0.f};
-        for (int j = 0; j < a.dims; ++j) acc = acc + imul(kap_d(a, m, j), ph[j * a.Nr]);
-        r = (-0.5f * a.scale) * acc;
-        break;
-      }
-      case NL_CONV_NONCONS:
-      case NL_VORT: r = -a.scale * ph[0]; break;
-      case NL_GENERAL: {
-        const float cg = (a.zero_mode_fix && m.zero) ? 0.f : 0.5f * a.g2;
-        r = a.g0 * ph[0] + imul(0.5f * a.g1 * (m.kx + m.ky + m.kz), ph[0]) + cg * ph[a.Nr];
-        break;
-      }
-      case NL_PROJ3D: {
-        // Leray projection (_leray.py:86-103): c + i kappa_c p with
-        // p = -div / Laplace = (i kappa . c) / |kappa|^2 (p = 0 at the mean mode)
-        const long long b = (inst - inst % a.channels) * a.Nr + k;  // np = 1
-        const cf p0 = PH[b], p1 = PH[b + a.Nr], p2 = PH[b + 2 * a.Nr];
-        const cf div = imul(m.kx, p0) + imul(m.ky, p1) + imul(m.kz, p2);
-        const float k2 = m.kx * m.kx + m.ky * m.ky + m.kz * m.kz;
-        const cf pr = k2 != 0.f ? (1.f / k2) * div : cf{0.f, 0.f};
-        const int c = (int)(inst % a.channels);
-        r = ph[0] + imul(c == 0 ? m.kx : c == 1 ? m.ky : m.kz, pr);
-        break;
-      }
-      default: r = ph[0];
-    }
-    cf out = m.keep ? r : cf{0.f, 0.f};
-    if ((a.kind == NL_PROJ3D || a.kind == NL_VORT) && m.inj && inst % a.channels == 0)
-      out = out + cf{a.inj_value, 0.f};
-    return out;
   }
 }
 
@@ -1340,96 +1230,6 @@ hipError_t launch_combine3d(const NL3DArgs& a, const cf* PH, cf* Nh, hipStream_t
 // coefficient c_i of the plan's tables (orders 1-2: [E, c1, c2] with Im E
 // at e_im for a complex L; order 3: 7 entries, order 4: 6, as coef.hip
 // forms them). X is the new state's spectrum.
-// Stages that read the first nonlinear term N0, and those that read the
-// latest one NC.
-__device__ __forceinline__ bool stage_reads_n0(int m) {
-  return m == ST1 || m == ST2A || m == ST2B || m == ST3A || m == ST3B || m == ST4A || m == ST4C;
-}
-__device__ __forceinline__ bool stage_reads_nc(int m) { return !(m == ST1 || m == ST2A || m == ST3A || m == ST4A); }
-
-// The coefficient table of instance (trajectory traj, channel ch).
-__device__ __forceinline__ const float* stage_table(const Stage3DArgs& a, long long traj, long long ch) {
-  return a.tables +
-         ((a.lin_batch > 1 ? traj : 0) * a.lin_channels + (a.lin_channels > 1 ? ch : 0)) * (long long)a.ncoef * a.nr;
-}
-
-// The stage combination of stage MODE at entry idx (mode k of its instance,
-// tb the instance's coefficient table) with the nonlinear terms n0 (N0) and
-// nc (NC) given; U0, S, S1, A as in Stage3DArgs. Returns the new S[idx].
-template <int MODE>
-__device__ __forceinline__ cf stage_core(int e_im, long long nr, const float* tb, long long k, long long idx,
-                                         const cf* U0, cf* S, cf* S1, cf* A, cf n0, cf nc) {
-  auto c = [&](int i) { return tb[(long long)i * nr + k]; };
-  // coefficient i (0: E, 1: E_half for orders 3-4) times x, complex when L is
-  auto cmul = [&](int i, cf x) -> cf {
-    const float er = c(i);
-    if (e_im < 0) return er * x;
-    const float ei = c(e_im + i);
-    return cf{fmaf(er, x.re, -ei * x.im), fmaf(er, x.im, ei * x.re)};
-  };
-  auto emul = [&](cf x) -> cf { return cmul(0, x); };
-  cf r;
-  if constexpr (MODE == ST1 || MODE == ST2A) {
-    r = emul(U0[idx]) + c(1) * n0;
-  } else if constexpr (MODE == ST2B) {
-    r = S[idx] + c(2) * (nc - n0);
-  } else if constexpr (MODE == ST3A) {
-    const cf u0 = U0[idx];
-    A[idx] = emul(u0) + c(4) * n0;
-    r = cmul(1, u0) + c(2) * n0;
-  } else if constexpr (MODE == ST3B) {
-    const cf u0 = U0[idx];
-    A[idx] = A[idx] + c(5) * nc;
-    r = emul(u0) + c(3) * (2.f * nc - n0);
-  } else if constexpr (MODE == ST3C) {
-    r = A[idx] + c(6) * nc;
-  } else if constexpr (MODE == ST4A) {
-    const cf u0 = U0[idx];
-    A[idx] = emul(u0) + c(3) * n0;
-    r = cmul(1, u0) + c(2) * n0;
-    S1[idx] = r;
-  } else if constexpr (MODE == ST4B) {
-    const cf u0 = U0[idx];
-    A[idx] = A[idx] + (2.f * c(4)) * nc;
-    r = cmul(1, u0) + c(2) * nc;
-  } else if constexpr (MODE == ST4C) {
-    A[idx] = A[idx] + (2.f * c(4)) * nc;
-    r = cmul(1, S1[idx]) + c(2) * (2.f * nc - n0);
-  } else {
-    static_assert(MODE == ST4D, "stage mode");
-    r = A[idx] + c(5) * nc;
-  }
-  S[idx] = r;
-  return r;
-}
-
-// Calls f(std::integral_constant<int, mode>) for the runtime stage mode.
-template <class F>
-__device__ __forceinline__ void with_stage_mode(int mode, F&& f) {
-  switch (mode) {
-    case ST1: f(std::integral_constant<int, ST1>{}); break;
-    case ST2A: f(std::integral_constant<int, ST2A>{}); break;
-    case ST2B: f(std::integral_constant<int, ST2B>{}); break;
-    case ST3A: f(std::integral_constant<int, ST3A>{}); break;
-    case ST3B: f(std::integral_constant<int, ST3B>{}); break;
-    case ST3C: f(std::integral_constant<int, ST3C>{}); break;
-    case ST4A: f(std::integral_constant<int, ST4A>{}); break;
-    case ST4B: f(std::integral_constant<int, ST4B>{}); break;
-    case ST4C: f(std::integral_constant<int, ST4C>{}); break;
-    case ST4D: f(std::integral_constant<int, ST4D>{}); break;
-  }
-}
-
-// The stage combination at entry idx with the nonlinear terms n0 (N0) and
-// nc (NC) given.
-__device__ __forceinline__ void stage_at(const Stage3DArgs& a, long long idx, cf n0, cf nc) {
-  const long long inst = idx / a.nr, k = idx % a.nr;
-  const float* tb = stage_table(a, inst / a.channels, inst % a.channels);
-  with_stage_mode(a.mode, [&](auto m) {
-    stage_core<decltype(m)::value>(a.e_im, a.nr, tb, k, idx, a.U0, a.S, a.S1, a.A, n0, nc);
-  });
-}
-
 __global__ void stage3d_kernel(Stage3DArgs a) {
   const long long total = a.ninst * a.nr;
   for (long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x; idx < total;
