@@ -41,11 +41,7 @@ constexpr int OW4 = OB3 + 32, OB4 = OW4 + 5120, OW5 = OB4 + 32, OB5 = OW5 + 160;
 constexpr int NPARAM = OB5 + 1;
 static_assert(NPARAM == 15809, "parameter count");
 constexpr int KSTEPS = CH * KW / 16;  // 10 MFMA K-steps per 32 -> 32 layer
-// packed fragments: 3 forward + 3 transposed hidden layers, then the forward
-// edge layers (layer 1: one K-step; layer 5: KSTEPS K-steps, row 0 only)
-constexpr int FRAG_L1 = 6 * KSTEPS * 64;
-constexpr int FRAG_L5 = FRAG_L1 + 64;
-constexpr int NFRAG = FRAG_L5 + KSTEPS * 64;
+constexpr int NFRAG = 3 * KSTEPS * 64;  // A fragments of the three hidden layers (one direction)
 constexpr int WAVES = 4;                // wavefronts per workgroup
 
 constexpr float GELU_C = 0.7978845608028654f;  // sqrt(2 / pi)
@@ -79,12 +75,14 @@ struct Edge {
   float w5[CH * KW];  // [ci][k]
   float b5;
   float bh[3][CH];  // b2, b3, b4
+  __attribute__((aligned(16))) __bf16 w5r[KW * CH];  // W5 as [k][ci]: row 0 of layer 5's A operand
 };
 
 __device__ inline void load_edge(Edge& e, const float* __restrict__ p) {
   for (int i = threadIdx.x; i < CH * KW; i += blockDim.x) {
     e.w1[i] = bf16r(p[OW1 + i]);
     e.w5[i] = bf16r(p[OW5 + i]);
+    e.w5r[(i % KW) * CH + i / KW] = static_cast<__bf16>(p[OW5 + i]);
   }
   for (int i = threadIdx.x; i < CH; i += blockDim.x) {
     e.b1[i] = p[OB1 + i];
@@ -95,26 +93,35 @@ __device__ inline void load_edge(Edge& e, const float* __restrict__ p) {
   if (threadIdx.x == 0) e.b5 = p[OB5];
 }
 
-// Packed fragment index of hidden layer L (0..2 = layers 2..4), K-step s,
-// lane l; T selects the transposed (input-gradient) operand.
-__host__ __device__ constexpr int frag_index(bool T, int L, int s, int l) {
-  return ((T ? 3 + L : L) * KSTEPS + s) * 64 + l;
+// Where weight (co, ci, k) of hidden layer L (0..2 = layers 2..4) lies in the
+// A fragments [layer][K-step][lane][8], as bfloat16 index; T: the transposed
+// (input-gradient) operand, rows ci and K = (k, co).
+template <bool T>
+__device__ __forceinline__ int frag_slot(int L, int co, int ci, int k) {
+  const int row = T ? ci : co, col = T ? co : ci;
+  return (((L * KSTEPS + 2 * k + (col >> 4)) * 64) + ((col >> 3) & 1) * 32 + row) * 8 + (col & 7);
+}
+
+// The A operand of layer 5 at K-step s: row 0 = W5, the other rows zero.
+__device__ __forceinline__ bf16x8 frag_l5(const Edge& e, int s, int lane) {
+  const bf16x8 v = *reinterpret_cast<const bf16x8*>(e.w5r + (s >> 1) * CH + (s & 1) * 16 + 8 * (lane >> 5));
+  return (lane & 31) == 0 ? v : bf16x8{};
 }
 
 // 32 x 32 output tiles t0 .. t0 + NTL - 1 (positions 32 t ..) of one hidden
 // layer from the activation rows `in` (shift +k - 2 forward, -k + 2
-// transposed). W: this layer's A fragments in LDS, [s][lane]. The tiles'
+// transposed). The tiles'
 // accumulation chains are interleaved to hide the MFMA dependency latency.
-template <int N, bool TRANSPOSED, int NTL>
-__device__ __forceinline__ void conv_tiles(f32x16 (&acc)[NTL], const bf16x8* W, const __bf16* in, int t0,
-                                           int lane) {
+// W(s): this lane's A operand of K-step s.
+template <int N, bool TRANSPOSED, int NTL, class A>
+__device__ __forceinline__ void conv_tiles(f32x16 (&acc)[NTL], A&& W, const __bf16* in, int t0, int lane) {
   const int c = lane & 31, h = lane >> 5;
 #pragma unroll
   for (int q = 0; q < NTL; ++q) acc[q] = f32x16{};
 #pragma unroll
   for (int s = 0; s < KSTEPS; ++s) {
     const int k = s >> 1;
-    const bf16x8 a = W[s * 64 + lane];
+    const bf16x8 a = W(s);
 #pragma unroll
     for (int q = 0; q < NTL; ++q) {
       const int p = ((t0 + q) * 32 + c + (TRANSPOSED ? 2 - k : k - 2)) & (N - 1);
@@ -141,15 +148,25 @@ __device__ __forceinline__ void wave_sync() {
 //   A0 bf16  [count][N]         rounded input
 //   A  bf16  [4][count][32][N]  activations a1..a4
 //   D  bf16  [4][count][32][N]  deltas (gradients of z1..z4)
+//   P  float [groups][NPARAM]   the weight-gradient pass's partial sums
 struct Workspace {
   float* Z;
   __bf16* A0;
   __bf16* A;
   __bf16* D;
+  float* P;
 };
 
+// Workgroups of the weight-gradient pass (per layer): one wavefront per
+// sample up to 128 of them; each writes one set of partial sums.
+__host__ __device__ inline int wgrad_groups(long long count) {
+  const long long g = (count + WAVES - 1) / WAVES;
+  return g < 128 ? (g < 1 ? 1 : (int)g) : 128;
+}
+
 __host__ __device__ inline long long workspace_bytes(int N, long long count) {
-  return count * N * (4LL * CH * 4 + 2 + 4LL * CH * 2 + 4LL * CH * 2);
+  const long long acts = count * N * (4LL * CH * 4 + 2 + 4LL * CH * 2 + 4LL * CH * 2);
+  return (acts + 15) / 16 * 16 + 4LL * wgrad_groups(count) * NPARAM;
 }
 
 __host__ __device__ inline Workspace workspace_at(void* base, int N, long long count) {
@@ -162,13 +179,11 @@ __host__ __device__ inline Workspace workspace_at(void* base, int N, long long c
   w.A = reinterpret_cast<__bf16*>(b);
   b += 4LL * count * CH * N * 2;
   w.D = reinterpret_cast<__bf16*>(b);
+  const long long acts = count * N * (4LL * CH * 4 + 2 + 4LL * CH * 2 + 4LL * CH * 2);
+  w.P = reinterpret_cast<float*>(static_cast<char*>(base) + (acts + 15) / 16 * 16);
   return w;
 }
 
-// Forward of one sample by one wavefront. xs: the sample's N inputs in LDS
-// (float); act0/act1: this wave's two activation buffers; the result
-// y = x + f(x) is written to y (global). With `ws` the training quantities
-// of sample `smp` are stored.
 // Bias, GELU and the bfloat16 activation rows of 32 x 32 output tiles
 // t0.. (layer index Lz of the training workspace).
 template <int N, bool TRAIN, int NTL>
@@ -200,12 +215,10 @@ __device__ __forceinline__ void act_epilogue(const f32x16 (&acc)[NTL], const flo
 // Forward of one sample by one wavefront. xs: the sample's N inputs in LDS
 // (float); act0/act1: this wave's two activation buffers (one and the same
 // when every output tile of a layer is formed before any is written); W: the hidden
-// layers' A fragments (LDS); F1, F5: the edge layers' A fragments (global,
-// cached); the result y = x + f(x) is written to y (global). With `ws` the
+// layers' A fragments (LDS); the result y = x + f(x) is written to y (global). With `ws` the
 // training quantities of sample `smp` are stored.
 template <int N, bool TRAIN>
-__device__ __forceinline__ void forward_sample(const Edge& e, const bf16x8* W, const bf16x8* F1, const bf16x8* F5,
-                                               const float* xs, __bf16* act0, __bf16* act1, float* __restrict__ y,
+__device__ __forceinline__ void forward_sample(const Edge& e, const bf16x8* W, const float* xs, __bf16* act0, __bf16* act1, float* __restrict__ y,
                                                Workspace ws, long long smp, long long count, int lane) {
   const int c = lane & 31, h = lane >> 5;
   constexpr int NTL = tiles_together<N>();
@@ -214,7 +227,9 @@ __device__ __forceinline__ void forward_sample(const Edge& e, const bf16x8* W, c
   }
   // layer 1 (1 -> 32): K = tap 0..4 (lanes of the upper half and taps >= 5 hold zeros)
   {
-    const bf16x8 a1 = F1[lane];
+    bf16x8 a1;  // A[co][K = tap]: taps 0..4 in the lower half's lanes, zeros elsewhere
+#pragma unroll
+    for (int i = 0; i < 8; ++i) a1[i] = static_cast<__bf16>(h == 0 && i < KW ? e.w1[c * KW + (i < KW ? i : 0)] : 0.f);
 #pragma unroll
     for (int t0 = 0; t0 < N / 32; t0 += NTL) {
       f32x16 acc[NTL];
@@ -241,7 +256,11 @@ __device__ __forceinline__ void forward_sample(const Edge& e, const bf16x8* W, c
 #pragma unroll
     for (int t0 = 0; t0 < N / 32; t0 += NTL) {
       f32x16 acc[NTL];
-      conv_tiles<N, false, NTL>(acc, W + L * KSTEPS * 64, in, t0, lane);
+      conv_tiles<N, false, NTL>(acc, [&](int s) { return W[(L * KSTEPS + s) * 64 + lane]; }, in, t0, lane);
+      // in place: a lane's own rows do not show that other lanes still read
+      // what it writes, so without the fence tile 0's writes may be moved
+      // before tile 1's reads
+      if (in == out) wave_sync();
       act_epilogue<N, TRAIN, NTL>(acc, e.bh[L], out, t0, lane, ws, smp, count, L + 1);
     }
     wave_sync();
@@ -253,7 +272,7 @@ __device__ __forceinline__ void forward_sample(const Edge& e, const bf16x8* W, c
 #pragma unroll
   for (int t0 = 0; t0 < N / 32; t0 += NTL) {
     f32x16 acc[NTL];
-    conv_tiles<N, false, NTL>(acc, F5, in, t0, lane);
+    conv_tiles<N, false, NTL>(acc, [&](int s) { return frag_l5(e, s, lane); }, in, t0, lane);
     if (h == 0) {
 #pragma unroll
       for (int q = 0; q < NTL; ++q) {
