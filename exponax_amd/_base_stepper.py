@@ -211,6 +211,36 @@ class BaseStepper:
                                           _lib.stream_ptr()), "exmi_repeat")
         return restore_like(out, back)
 
+    def _repeat_checkpointed(self, x, n: int, every: int):
+        """``repeat_batch`` of the contiguous float32 device batch ``x`` that
+        also returns the states after ``every``, 2 ``every``, ... < n steps
+        (exmi_repeat_checkpointed), for ``_repeat_vjp``."""
+        import torch
+
+        _, B = self._split(x, self.state_shape)
+        k = every if 0 < every < n else max(n, 1)
+        out = torch.empty_like(x)
+        ckpt = torch.empty((max(-(-n // k), 1) - 1,) + tuple(x.shape), dtype=torch.float32, device=x.device)
+        p = self.plan(B)
+        _lib.check(_lib.lib().exmi_repeat_checkpointed(p.handle, x.data_ptr(), x.numel() // B, out.data_ptr(),
+                                                       ckpt.data_ptr(), n, int(every), _lib.stream_ptr()),
+                   "exmi_repeat_checkpointed")
+        return out, ckpt
+
+    def _repeat_vjp(self, x, n: int, ckpt, g, every: int):
+        """Gradient of ``repeat_batch`` from the checkpoints of its forward
+        pass (exmi_repeat_vjp)."""
+        import torch
+
+        _, B = self._split(x, self.state_shape)
+        g = g.contiguous().to(torch.float32)
+        out = torch.empty_like(x)
+        p = self.plan(B)
+        _lib.check(_lib.lib().exmi_repeat_vjp(p.handle, x.data_ptr(), x.numel() // B, n, ckpt.data_ptr(),
+                                              g.data_ptr(), out.data_ptr(), int(every), _lib.stream_ptr()),
+                   "exmi_repeat_vjp")
+        return out
+
     # --------------------------------------------------------- derivatives
     def step_vjp(self, u, g):
         """(d step(u) / d u)^T g for one state or a batch (the reverse-mode

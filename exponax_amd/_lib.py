@@ -45,7 +45,7 @@ EXPORTED = (
     "exmi_map_resolution", "exmi_ic_tfs", "exmi_wave_step_fourier", "exmi_poisson_fourier", "exmi_axpy",
     "exmi_cnn_workspace_bytes", "exmi_cnn_forward", "exmi_cnn_backward", "exmi_corrected_rollout",
     "exmi_irfft_noalloc", "exmi_rollout_checked", "exmi_first_bad_step", "exmi_plan_fft_config",
-    "exmi_plan_set_fft_config",
+    "exmi_plan_set_fft_config", "exmi_repeat_checkpointed", "exmi_repeat_vjp",
 )
 EXMI_NOALLOC_SCRATCH_BYTES = 32 << 20
 EXMI_CNN_NUM_PARAMS = 15809
@@ -104,6 +104,8 @@ def _declare(lib):
     lib.exmi_rollout_group.argtypes = [C.POINTER(vp), i32, C.POINTER(vp), C.POINTER(i64), C.POINTER(vp), i32, i32,
                                        i32, vp]
     lib.exmi_repeat.argtypes = [vp, vp, i64, vp, i32, i32, vp]
+    lib.exmi_repeat_checkpointed.argtypes = [vp, vp, i64, vp, vp, i32, i32, vp]
+    lib.exmi_repeat_vjp.argtypes = [vp, vp, i64, i32, vp, vp, vp, i32, vp]
     lib.exmi_rfft.argtypes = [i32, i32, i32, vp, vp, vp]
     lib.exmi_irfft.argtypes = [i32, i32, i32, vp, vp, vp]
     lib.exmi_irfft_noalloc.argtypes = [i32, i32, i32, vp, vp, vp]

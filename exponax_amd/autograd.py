@@ -3,8 +3,9 @@ whose backward passes run the hand-written adjoint kernels.
 
 The reference gets its derivatives from ``jax.grad`` through ``lax.scan``
 (``_utils.py:92-254``, README.md:85-91). It keeps every step's residuals. Here
-the backward of a rollout keeps one state every ``checkpoint_every`` steps
-and recomputes each segment on the way back.
+one state every ``checkpoint_every`` steps is kept (by the forward pass of
+``repeat``, by the backward of ``rollout``) and each segment is recomputed on
+the way back.
 
     u0 = torch.randn(32, 1, 128, 128, device="cuda", requires_grad=True)
     uT = exponax_amd.autograd.repeat(stepper, u0, 50, checkpoint_every=10)
@@ -14,6 +15,8 @@ and recomputes each segment on the way back.
 from __future__ import annotations
 
 import torch
+
+from ._base_stepper import BaseStepper
 
 
 class _Step(torch.autograd.Function):
@@ -48,11 +51,23 @@ class _Repeat(torch.autograd.Function):
     @staticmethod
     def forward(ctx, u0, stepper, n, checkpoint_every):
         ctx.stepper, ctx.n, ctx.k = stepper, n, checkpoint_every
+        # the checkpoints the backward starts its segments from are states
+        # this pass goes through: kept here, the backward need not run it again
+        ctx.keep = (ctx.needs_input_grad[0] and n > checkpoint_every > 0 and isinstance(stepper, BaseStepper)
+                    and getattr(stepper, "_groups", None) is None and u0.dtype == torch.float32
+                    and u0.is_contiguous())
+        if ctx.keep:
+            out, ckpt = stepper._repeat_checkpointed(u0.detach(), n, checkpoint_every)
+            ctx.save_for_backward(u0, ckpt)
+            return out
         ctx.save_for_backward(u0)
         return stepper.repeat_batch(u0.detach(), n)
 
     @staticmethod
     def backward(ctx, g):
+        if ctx.keep:
+            u0, ckpt = ctx.saved_tensors
+            return ctx.stepper._repeat_vjp(u0.detach(), ctx.n, ckpt, g, ctx.k), None, None, None
         (u0,) = ctx.saved_tensors
         return ctx.stepper.rollout_vjp(u0.detach(), ctx.n, g_final=g.contiguous(), checkpoint_every=ctx.k), None, \
             None, None

@@ -2631,6 +2631,10 @@ static int effective_nt(const exmi_plan* p) {
   return p->roll[2] ? 2 : (p->roll[1] ? 1 : -1);
 }
 
+// Steps per segment of a rollout gradient (checkpoint_every <= 0 or >= n:
+// one segment).
+static int vjp_segment(int n, int every) { return every > 0 && every < n ? every : (n > 0 ? n : 1); }
+
 static int enq_repeat_cb(exmi_plan* p, const void* a, const void* b, long long s, int n, int, hipStream_t st) {
   const float* u0 = (const float*)a;
   float* out = (float*)b;
@@ -2902,6 +2906,26 @@ int exmi_repeat(exmi_plan* p, const float* u0, int64_t u0_bs, float* u_out, int3
     if (rc) return rc;
   }
   return run_maybe_graph(p, u0, u_out, u0_bs, n, 0, 2, use_graph, (hipStream_t)stream, enq_repeat_cb);
+}
+
+int exmi_repeat_checkpointed(exmi_plan* p, const float* u0, int64_t u0_bs, float* u_out, float* ckpt, int32_t n,
+                             int32_t every, void* stream) {
+  if (!p || !u0 || !u_out) return fail(EXMI_ERR_INVALID, "null argument");
+  if (n < 0) return fail(EXMI_ERR_INVALID, "n_steps must be >= 0");
+  const int K = vjp_segment(n, every), nseg = n > 0 ? (n + K - 1) / K : 1;
+  if (nseg > 1 && !ckpt) return fail(EXMI_ERR_INVALID, "null argument");
+  if (K > 1) {
+    int rc = ensure_work(p);
+    if (rc) return rc;
+  }
+  const long long sz = state_size(p), bsz = (long long)p->d.batch * sz;
+  for (int s = 0; s < nseg; ++s) {
+    const float* in = s == 0 ? u0 : ckpt + (s - 1) * bsz;
+    float* out = s == nseg - 1 ? u_out : ckpt + s * bsz;
+    int rc = enq_repeat_cb(p, in, out, s == 0 ? u0_bs : sz, n - s * K < K ? n - s * K : K, 0, (hipStream_t)stream);
+    if (rc) return rc;
+  }
+  return EXMI_OK;
 }
 
 }  // extern "C"
@@ -3409,9 +3433,11 @@ int exmi_step_vjp(exmi_plan* p, const float* u, int64_t u_bs, const float* g, in
   return enqueue_step_vjp(p, u, u_bs, g, g_bs, g_in, gin_bs, (hipStream_t)stream);
 }
 
-int exmi_rollout_vjp(exmi_plan* p, const float* u0, int64_t u0_bs, int32_t n, int32_t include_init,
-                     const float* g_traj, const float* g_final, float* g_u0, int32_t checkpoint_every,
-                     void* stream) {
+// given: the states after K, 2 K, ... steps from a checkpointed forward pass
+// (exmi_repeat_checkpointed), or null: formed here.
+static int rollout_vjp(exmi_plan* p, const float* u0, int64_t u0_bs, int32_t n, int32_t include_init,
+                       const float* g_traj, const float* g_final, float* g_u0, int32_t checkpoint_every,
+                       const float* given, void* stream) {
   if (!p || !u0 || !g_u0) return fail(EXMI_ERR_INVALID, "null argument");
   if (n < 0) return fail(EXMI_ERR_INVALID, "n_steps must be >= 0");
   if (!has_adjoint(p))
@@ -3422,13 +3448,14 @@ int exmi_rollout_vjp(exmi_plan* p, const float* u0, int64_t u0_bs, int32_t n, in
   const long long bsz = (long long)B * sz;
   const int off = include_init ? 1 : 0;
   const long long gts = (long long)(n + off) * sz;  // g_traj batch stride
-  int K = checkpoint_every > 0 && checkpoint_every < n ? checkpoint_every : (n > 0 ? n : 1);
+  const int K = vjp_segment(n, checkpoint_every);
   const int nseg = n > 0 ? (n + K - 1) / K : 0;
   int rc = ensure_adjoint_ws(p);
   if (!rc) rc = ensure_work(p);
   if (rc) return rc;
-  // workspace: nseg checkpoints (B, sz) | one segment (B, K, sz) | accumulator (B, sz)
-  const size_t need = (size_t)((long long)nseg * bsz + (long long)K * bsz + bsz);
+  // workspace: nseg checkpoints (B, sz), unless given | one segment (B, K, sz) | accumulator (B, sz)
+  const int nown = given ? 0 : nseg;
+  const size_t need = (size_t)((long long)nown * bsz + (long long)K * bsz + bsz);
   if (p->ckpt_elems < need) {
     HIP_TRY(hipStreamSynchronize(st));
     hipFree(p->ckpt);
@@ -3452,15 +3479,17 @@ int exmi_rollout_vjp(exmi_plan* p, const float* u0, int64_t u0_bs, int32_t n, in
     p->gseg_elems = K * gblk;
   }
   float* cp = p->ckpt;
-  float* seg = cp + (long long)nseg * bsz;
+  float* seg = cp + (long long)nown * bsz;
   float* acc = seg + (long long)K * bsz;
   hipError_t e = g_final ? copy_batch(g_final, sz, acc, sz, sz, B, st) : fill(acc, bsz, 0.f, st);
   if (e != hipSuccess) return fail(EXMI_ERR_HIP, "launch failed: %s", hipGetErrorString(e));
   if (n > 0) {
     // forward pass keeping every K-th state
-    e = copy_batch(u0, u0_bs, cp, sz, sz, B, st);
-    if (e != hipSuccess) return fail(EXMI_ERR_HIP, "launch failed: %s", hipGetErrorString(e));
-    for (int sidx = 1; sidx < nseg; ++sidx) {
+    if (!given) {
+      e = copy_batch(u0, u0_bs, cp, sz, sz, B, st);
+      if (e != hipSuccess) return fail(EXMI_ERR_HIP, "launch failed: %s", hipGetErrorString(e));
+    }
+    for (int sidx = 1; sidx < nown; ++sidx) {
       rc = enq_repeat_cb(p, cp + (long long)(sidx - 1) * bsz, cp + (long long)sidx * bsz, sz, K, 0, st);
       if (rc) return rc;
     }
@@ -3468,14 +3497,16 @@ int exmi_rollout_vjp(exmi_plan* p, const float* u0, int64_t u0_bs, int32_t n, in
     for (int sidx = nseg - 1; sidx >= 0; --sidx) {
       const int t0 = sidx * K;
       const int len = (n - t0) < K ? (n - t0) : K;
+      const float* from = !given ? cp + (long long)sidx * bsz : sidx == 0 ? u0 : given + (long long)(sidx - 1) * bsz;
+      const long long fbs = given && sidx == 0 ? u0_bs : sz;
       if (coop) {
         // the segment's len steps as one cooperative launch that keeps the
         // gradient fields of every step (its states are not needed; the last
         // one lands in seg), then the transposed steps from those fields
-        rc = enqueue_coop2d(p, cp + (long long)sidx * bsz, sz, seg, sz, 0, len, 1, st, p->Gseg, gblk);
+        rc = enqueue_coop2d(p, from, fbs, seg, sz, 0, len, 1, st, p->Gseg, gblk);
         if (rc) return rc;
       } else {
-        rc = enqueue_rollout_nt(p, effective_nt(p), cp + (long long)sidx * bsz, sz, seg, len - 1, 1, st);
+        rc = enqueue_rollout_nt(p, effective_nt(p), from, fbs, seg, len - 1, 1, st);
         if (rc) return rc;
       }
       const long long segs = (long long)len * sz;  // segment batch stride
@@ -3522,6 +3553,18 @@ int exmi_rollout_vjp(exmi_plan* p, const float* u0, int64_t u0_bs, int32_t n, in
   }
   e = copy_batch(acc, sz, g_u0, sz, sz, B, st);
   return e == hipSuccess ? EXMI_OK : fail(EXMI_ERR_HIP, "launch failed: %s", hipGetErrorString(e));
+}
+
+int exmi_rollout_vjp(exmi_plan* p, const float* u0, int64_t u0_bs, int32_t n, int32_t include_init,
+                     const float* g_traj, const float* g_final, float* g_u0, int32_t checkpoint_every,
+                     void* stream) {
+  return rollout_vjp(p, u0, u0_bs, n, include_init, g_traj, g_final, g_u0, checkpoint_every, nullptr, stream);
+}
+
+int exmi_repeat_vjp(exmi_plan* p, const float* u0, int64_t u0_bs, int32_t n, const float* ckpt, const float* g_final,
+                    float* g_u0, int32_t checkpoint_every, void* stream) {
+  if (!g_final || (!ckpt && n > vjp_segment(n, checkpoint_every))) return fail(EXMI_ERR_INVALID, "null argument");
+  return rollout_vjp(p, u0, u0_bs, n, 0, nullptr, g_final, g_u0, checkpoint_every, ckpt, stream);
 }
 
 }  // extern "C"
