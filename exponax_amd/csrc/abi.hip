@@ -1168,14 +1168,19 @@ static bool zprod_kind(const exmi_plan* p) {
           k3 == NL_CONV_CONS || k3 == NL_CONV_NONCONS);
 }
 
-// Fused 3-D plans whose forward x lines run with the combine and the stage
-// (xstage3d_kernel, xstage_proj3d_kernel) inside an ETDRK step.
+// Plans whose last forward axis runs with the combine and the stage inside
+// an ETDRK step: the fused 3-D sizes (xstage3d_kernel, xstage_proj3d_kernel),
+// and the runtime sizes whose lines fit LDS (gstage_kernel).
+static bool gen_fused(const exmi_plan* p, const NL3DArgs& a) {
+  return p->gen && p->ndim >= 2 && p->kmax >= 0 && gprod_fits(p->gcfg, a);
+}
+static bool gen_stage(const exmi_plan* p, const NL3DArgs& a) { return gen_fused(p, a) && gstage_fits(p->gcfg, a); }
 static bool xstage_kind(const exmi_plan* p) {
   return zprod_kind(p) || (!p->gen && p->kind3 == NL_PROJ3D && p->d.num_points <= 128);
 }
 
 // The product spectra of N(X) of every instance into F3 (the passes of
-// spectral3d.hip up to the combine).
+// spectral3d.hip and gspec.hip up to the combine).
 // *ph: where the product spectra are (F3, or for the projected convection
 // of a fused size R3 as spectra). no_x: the forward x lines of the kinds
 // with fused z rows are left to the caller (stages3d fuses them with the
@@ -1183,7 +1188,7 @@ static bool xstage_kind(const exmi_plan* p) {
 static hipError_t nonlinear3d_products(exmi_plan* p, const NL3DArgs& a, const cf* X, hipStream_t st,
                                        const cf** ph, bool no_x = false) {
   *ph = p->F3;
-  if (p->gen && p->ndim >= 2 && p->kmax >= 0 && gprod_fits(p->gcfg, a)) {
+  if (gen_fused(p, a)) {
     // the fields with the first inverse axis, the rows with the products, and
     // the forward axes; what the dealias cutoff makes zero or the combine
     // does not read is left out
@@ -1200,7 +1205,7 @@ static hipError_t nonlinear3d_products(exmi_plan* p, const NL3DArgs& a, const cf
       e = launch_gfft(p->gcfg, GFFT_INV, p->F3, p->F3, y, r, tw, st);
     }
     if (e == hipSuccess) e = launch_gprod(p->gcfg, a, p->F3, P, r, kk, tw, st);
-    for (int ax = p->ndim - 2; ax >= 0 && e == hipSuccess; --ax) {
+    for (int ax = p->ndim - 2; ax >= (no_x ? 1 : 0) && e == hipSuccess; --ax) {
       GfftLines g = axis_lines(p->ndim, ax, N, p->ninst * p->np3);
       g.kkeep = kk;
       g.cut = g.pcut = cut;
@@ -1309,7 +1314,7 @@ static hipError_t stages3d(exmi_plan* p, Stage3DArgs& sa, hipStream_t st, cf* em
   NL3DArgs a;
   fill_nl3d(p, a);
   const int N = p->d.num_points, NZ = N / 2 + 1;
-  const bool xs = xstage_kind(p);
+  const bool gs = gen_stage(p, a), xs = xstage_kind(p);
   const int kz = p->kmax < NZ - 1 ? (p->kmax < 0 ? 0 : p->kmax) : NZ - 1;
   const bool em = emitK && xs;
   if (emitted) *emitted = em;
@@ -1319,11 +1324,12 @@ static hipError_t stages3d(exmi_plan* p, Stage3DArgs& sa, hipStream_t st, cf* em
     if (m < 0) break;
     const bool last = i == 3 || seq[p->d.order - 1][i + 1] < 0;
     const cf* ph = nullptr;
-    e = nonlinear3d_products(p, a, i == 0 ? sa.U0 : sa.S, st, &ph, xs);
+    e = nonlinear3d_products(p, a, i == 0 ? sa.U0 : sa.S, st, &ph, xs || gs);
     sa.mode = m;
     cf* n0 = i == 0 ? p->N03 : nullptr;
     if (e == hipSuccess)
-      e = !xs                          ? launch_stage_nl3d(a, sa, ph, n0, st)
+      e = gs ? launch_gstage(p->gcfg, a, sa, ph, n0, kz + 1, p->kmax < N ? p->kmax : N, p->tw_col.tw, st)
+          : !xs                        ? launch_stage_nl3d(a, sa, ph, n0, st)
           : p->kind3 == NL_PROJ3D ? launch_xstage_proj3d(a, sa, ph, n0, kz, p->tw_col.tw, st,
                                                          em && last ? emitK : nullptr)
                                   : launch_xstage3d(a, sa, ph, n0, kz, p->tw_col.tw, st, em && last ? emitK : nullptr);

@@ -18,7 +18,7 @@
 // by runtime sizes are float multiplications; the lines of a workgroup share
 // their twiddle reads and lie side by side at an odd pitch.
 // Measured (eight 513^2 fields, one transform along one axis): forward lines
-// 22 us, inverse lines 19 us, r2c 20 us, c2r 15 us, against 33, 33, 42 and
+// 15 us, inverse lines 13 us, r2c 18 us, c2r 15 us, against 33, 33, 42 and
 // 43 us with one real line per transform, R^2 complex products per radix-R
 // butterfly and integer divisions; a prime pass of 199 points (N = 597, one
 // step of 100 trajectories) 60 us per step against 185 us with direct sums.
@@ -47,7 +47,7 @@ __global__ void __launch_bounds__(GFFT_WG) gfft_kernel(GfftArgs a) {
   constexpr bool INV = MODE == GFFT_INV || MODE == GFFT_C2R;
   constexpr bool REAL = MODE == GFFT_R2C || MODE == GFFT_C2R;
   const int n = a.d.n, nz = n / 2 + 1, tid = threadIdx.x;
-  const long long run0 = (long long)blockIdx.x * a.lpb;
+  const long long run0 = (long long)(REAL ? blockIdx.x : xcd_block()) * a.lpb;
   const int L = (int)(a.nrun - run0 < a.lpb ? a.nrun - run0 : a.lpb);
   const int pitch = gfft_pitch(a.lpb);
   cf* A = gfft_smem;

@@ -2,11 +2,13 @@
 // set) around the line transforms of gfft.hpp: the spectral fields with the
 // first inverse axis, the rows of the last axis with the pointwise products,
 // and in 1-D whole ETDRK rollouts in one launch.
-// One nonlinear evaluation of eight 513^2 Kolmogorov instances: 33 us of
-// fields, 45 us of rows and products, 17 us of forward lines and 13 us of
-// stage, against 358 us as separate fields, transforms of whole fields
-// (119 + 88 us for the four fields), products, transforms and stage. What
-// bounds the two fused passes is the instruction issue of the butterflies.
+// One nonlinear evaluation of eight 513^2 Kolmogorov instances: 28 us of
+// fields, 46 us of rows and products, 25 us of forward lines with the stage,
+// against 358 us as separate fields, transforms of whole fields (119 + 88 us
+// for the four fields), products, transforms and stage. What bounds them is
+// the latency of the short passes between barriers at three to five
+// workgroups per CU; passes in place in registers (half the LDS, twice the
+// barriers) gave 42 us for the rows at 513 and cost 8% of a step at 48^3.
 #include "gspec.hpp"
 #include "nl3d.hpp"
 
@@ -35,7 +37,7 @@ __global__ void __launch_bounds__(GFFT_WG) gfields_kernel(GFieldsArgs g) {
   __shared__ int bf[GFFT_MAX_LINES], bm[GFFT_MAX_LINES], bz[GFFT_MAX_LINES];
   __shared__ long long bi[GFFT_MAX_LINES];
   const int n = g.d.n, tid = threadIdx.x;
-  const long long run0 = (long long)blockIdx.x * g.lpb;
+  const long long run0 = (long long)xcd_block() * g.lpb;
   const int L = (int)(g.nrun - run0 < g.lpb ? g.nrun - run0 : g.lpb);
   const int pitch = gfft_pitch(g.lpb);
   cf* A = gspec_smem;
@@ -224,6 +226,128 @@ hipError_t launch_gprod(const GfftCfg& c, const NL3DArgs& a, const cf* F, cf* P,
   auto* k = gfft_big(c) ? (twl ? gprod_kernel<19, true> : gprod_kernel<19, false>)
                         : (twl ? gprod_kernel<8, true> : gprod_kernel<8, false>);
   hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(GFFT_WG), lds, st, g);
+  return hipGetLastError();
+}
+
+// -------------------------------------- last forward axis + combine + stage
+struct GStageArgs {
+  NL3DArgs a;
+  GfftDev d;
+  int units, npt, kkeep, midn, cut;  // lines (trajectory, m, kz) per workgroup; products per trajectory
+  long long nunits, pstride;
+  const cf* P;
+  cf* N0out;
+  const cf* tw;
+};
+
+// The combine and stage M at every point of the workgroup's U lines.
+template <int M>
+__device__ __forceinline__ void gstage_points(const GStageArgs& g, const Stage3DArgs& st, const cf* Z, const long long* b0, const int* bm,
+                                              const int* bz, const int* bk, int U, int pitch) {
+  const int C = g.a.channels, np = g.a.np, n = g.d.n;
+  const float rU = 1.f / (float)U, rC = 1.f / (float)C;
+  for (int idx = threadIdx.x; idx < U * C * n; idx += GFFT_WG) {
+    const int q = fdiv(idx, rU), u = idx - q * U, pt = fdiv(q, rC), c = q - pt * C;
+    const Mode3D md = g.midn > 1 ? mode3d_at(g.a, pt, bm[u], bz[u]) : mode3d_at(g.a, 0, pt, bz[u]);
+    const cf* z = Z + pt * pitch + u;
+    const int keep = bk[u];
+    const cf nh = combine_core(g.a, md, c, [=](int cc, int j) { return keep ? z[(cc * np + j) * U] : cf{0.f, 0.f}; });
+    const long long k = pt * g.pstride + (long long)bm[u] * g.a.NZ + bz[u];
+    const long long at = (b0[u] * C + c) * g.a.Nr + k;
+    cf n0 = nh;
+    if (g.N0out) g.N0out[at] = nh;
+    else if (stage_reads_n0(M)) n0 = st.N0[at];
+    stage_core<M>(st.e_im, st.nr, stage_table(st, b0[u], c), k, at, st.U0, st.S, st.S1, st.A, n0, nh);
+  }
+}
+
+// The products' lines of the outermost axis, transformed and then combined
+// into N_hat and the stage at every point while they are in LDS: neither the
+// product spectra's last pass nor a combine pass goes through memory: 25 us
+// for eight 513^2 instances, 17 + 13 us as two passes. Lines beyond the
+// dealias cutoff hold no products; their N_hat is zero. The stage's arguments
+// are a kernel parameter of their own: inside the other struct its ten-way
+// switch made the compiler copy all arguments to scratch (44 us).
+template <int RMAX, bool TWL>
+__global__ void __launch_bounds__(GFFT_WG) gstage_kernel(GStageArgs g, Stage3DArgs st) {
+  extern __shared__ cf gspec_smem[];
+  __shared__ long long b0[GFFT_MAX_LINES];  // trajectory
+  __shared__ int bm[GFFT_MAX_LINES], bz[GFFT_MAX_LINES], bk[GFFT_MAX_LINES];
+  const int n = g.d.n, tid = threadIdx.x;
+  const long long u0 = (long long)xcd_block() * g.units;
+  const int U = (int)(g.nunits - u0 < g.units ? g.nunits - u0 : g.units);
+  const int L = U * g.npt, pitch = gfft_pitch(g.units * g.npt);
+  cf* A = gspec_smem;
+  cf* B = gspec_smem + n * pitch;
+  const cf* T = TWL ? gspec_smem + 2 * n * pitch : g.tw;
+  if constexpr (TWL)
+    for (int i = tid; i < n; i += GFFT_WG) gspec_smem[2 * n * pitch + i] = g.tw[i];
+  if (tid < U) {
+    const long long unit = u0 + tid, r = unit / g.a.NZ, b = r / g.midn;
+    const int z = (int)(unit - r * g.a.NZ), m = (int)(r - b * g.midn);
+    b0[tid] = b;
+    bm[tid] = m;
+    bz[tid] = z;
+    bk[tid] = z < g.kkeep && (g.midn == 1 || m <= g.cut || g.midn - m <= g.cut);
+  }
+  __syncthreads();
+  bool any = false;
+  for (int u = 0; u < U; ++u) any = any || bk[u];
+  const float rL = 1.f / (float)L, rU = 1.f / (float)U;
+  const cf* Z = A;
+  if (any) {
+    for (int idx = tid; idx < L * n; idx += GFFT_WG) {
+      const int pt = fdiv(idx, rL), l = idx - pt * L;  // line l = j * U + u: neighbouring threads, neighbouring kz
+      const int j = fdiv(l, rU), u = l - j * U;
+      A[pt * pitch + l] = bk[u] ? g.P[(b0[u] * g.npt + j) * g.a.Nr + pt * g.pstride + (long long)bm[u] * g.a.NZ + bz[u]]
+                                : cf{0.f, 0.f};
+    }
+    __syncthreads();
+    Z = gfft_run<false, RMAX>(A, B, T, g.d, L, pitch, tid, GFFT_WG);
+  }
+  switch (st.mode) {
+#define EXMI_GSTAGE(M) \
+  case M: gstage_points<M>(g, st, Z, b0, bm, bz, bk, U, pitch); break;
+    EXMI_GSTAGE(ST1) EXMI_GSTAGE(ST2A) EXMI_GSTAGE(ST2B) EXMI_GSTAGE(ST3A) EXMI_GSTAGE(ST3B) EXMI_GSTAGE(ST3C)
+    EXMI_GSTAGE(ST4A) EXMI_GSTAGE(ST4B) EXMI_GSTAGE(ST4C) EXMI_GSTAGE(ST4D)
+#undef EXMI_GSTAGE
+  }
+}
+
+static size_t gstage_lds(int n, int npt, int units, bool tw) {
+  return sizeof(cf) * ((size_t)2 * n * gfft_pitch(units * npt) + (tw ? n : 0));
+}
+constexpr size_t GSTAGE_FIXED = 20 * GFFT_MAX_LINES;
+
+bool gstage_fits(const GfftCfg& c, const NL3DArgs& a) {
+  return a.dims >= 2 && gstage_lds(c.n, a.channels * a.np, 1, false) + GSTAGE_FIXED <= GFFT_LDS_MAX;
+}
+
+hipError_t launch_gstage(const GfftCfg& c, const NL3DArgs& a, const Stage3DArgs& sa, const cf* P, cf* N0out,
+                         int kkeep, int cut, const cf* tw, hipStream_t st) {
+  if (!gstage_fits(c, a) || c.n != a.N || kkeep < 1 || kkeep > a.NZ) return hipErrorInvalidValue;
+  GStageArgs g;
+  g.a = a;
+  g.d = gfft_dev(c);
+  g.npt = a.channels * a.np;
+  g.units = c.lpb / g.npt;
+  if (g.units < 1) g.units = 1;
+  while (g.units > 1 && gstage_lds(c.n, g.npt, g.units, false) + GSTAGE_FIXED > GFFT_LDS_MAX) --g.units;
+  g.kkeep = kkeep;
+  g.cut = cut;
+  g.midn = a.dims == 3 ? a.ny : 1;
+  g.pstride = a.dims == 3 ? (long long)a.ny * a.NZ : a.NZ;
+  g.nunits = a.ninst / a.channels * g.midn * a.NZ;
+  g.P = P;
+  g.N0out = N0out;
+  g.tw = tw;
+  const long long grid = (g.nunits + g.units - 1) / g.units;
+  if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
+  const bool twl = gstage_lds(c.n, g.npt, g.units, true) + GSTAGE_FIXED <= GFFT_LDS_MAX;
+  const size_t lds = gstage_lds(c.n, g.npt, g.units, twl);
+  auto* k = gfft_big(c) ? (twl ? gstage_kernel<19, true> : gstage_kernel<19, false>)
+                        : (twl ? gstage_kernel<8, true> : gstage_kernel<8, false>);
+  hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(GFFT_WG), lds, st, g, sa);
   return hipGetLastError();
 }
 

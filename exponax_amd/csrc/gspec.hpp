@@ -19,6 +19,13 @@ bool gprod_fits(const GfftCfg& c, const NL3DArgs& a);
 hipError_t launch_gprod(const GfftCfg& c, const NL3DArgs& a, const cf* F, cf* P, float scale, int kkeep,
                         const cf* tw, hipStream_t st);
 
+// The last forward axis of the products P (2-D and 3-D) with the combine and
+// the stage st (N0out: also store N_hat, the first stage's): lines kz < kkeep
+// and, in 3-D, |ky| <= cut hold products.
+bool gstage_fits(const GfftCfg& c, const NL3DArgs& a);
+hipError_t launch_gstage(const GfftCfg& c, const NL3DArgs& a, const Stage3DArgs& st, const cf* P, cf* N0out,
+                         int kkeep, int cut, const cf* tw, hipStream_t stream);
+
 // 1-D: `nsteps` whole ETDRK steps (orders 0-4) of every trajectory in one launch.
 struct G1dArgs {
   NL3DArgs nl;
