@@ -399,7 +399,7 @@ struct exmi_plan {
   Twiddles tw;
   StepFn step = nullptr;
   StepFn nonlin = nullptr;
-  RollFn roll[3] = {nullptr, nullptr, nullptr};  // by transforms per lane group (1, 2)
+  RollFn roll[4] = {};  // by transforms per lane group (1, 2); 3: one on twice the lanes
   int roll_nt = 0;                               // chosen by the autotuner (0 = not yet)
   int tune_short = 0;  // chosen on a probe shorter than kTuneProbe steps: timed again on a longer rollout
   int fourier_resident = 0;                      // rollouts keep the spectral state on chip
@@ -1962,6 +1962,7 @@ int exmi_plan_create(const exmi_plan_desc* d, exmi_plan** out) {
               : cplx  ? get_roll1d_c(p->M, kind, d->order, fr)
                       : get_roll1d(p->M, kind, d->order, 1, fr, std_kc);
   p->roll[2] = (cplx || coupled) ? nullptr : get_roll1d(p->M, kind, d->order, 2, fr, std_kc);
+  p->roll[3] = (cplx || coupled) ? nullptr : get_roll1d(p->M, kind, d->order, 3, fr, std_kc);
   if (const char* e = getenv("EXMI_ROLL_NT")) p->roll_nt = atoi(e);  // 1, 2; -1 = per-step launches
   if (p->fourier_resident && !p->fr_auto && p->roll_nt < 0) p->roll_nt = 0;
   if (coupled) {
@@ -2076,7 +2077,7 @@ static bool strategy_ok(const exmi_plan* p, int nt) {
   if (nt == -1) return !(p->fourier_resident && !p->fr_auto);
   if (p->md) return nt == 2 && p->md_carry;
   if (p->ndim == 2) return (nt == 1 && p->roll2d != nullptr) || (nt == 2 && p->fr2d) || (nt == 3 && p->coop2d);
-  return (nt == 1 || nt == 2) && p->roll[nt] != nullptr;
+  return nt >= 1 && nt <= 3 && p->roll[nt] != nullptr;
 }
 
 int exmi_plan_rollout_strategy(const exmi_plan* p) { return p ? p->roll_nt : fail(EXMI_ERR_INVALID, "null plan"); }
@@ -2634,6 +2635,8 @@ static int effective_nt(const exmi_plan* p) {
     if (p->coop2d) return 3;
     return p->fr2d ? 2 : -1;
   }
+  // 1-D: the latency variant while it needs no more wavefronts than there are SIMDs
+  if (p->roll[3] && (long long)p->d.batch * p->d.num_channels * (p->M / 4) <= 1024 * 64LL) return 3;
   return p->roll[2] ? 2 : (p->roll[1] ? 1 : -1);
 }
 
@@ -2777,7 +2780,9 @@ int exmi_rollout_checked(exmi_plan* p, const float* u0, int64_t u0_bs, float* tr
 // and, beside the other members' launches on concurrent streams, slowed
 // the mixed Kolmogorov batch (32 x 128^2 + 16 x 256^2 + 8 x 512^2: 99.4
 // against 86-92 us per step).
-static int member_nt(const exmi_plan* p, int np) { return (np > 1 && p->roll_nt == 3) ? 2 : p->roll_nt; }
+static int member_nt(const exmi_plan* p, int np) {
+  return (np > 1 && p->ndim == 2 && p->roll_nt == 3) ? 2 : p->roll_nt;
+}
 
 static int enqueue_member(exmi_plan* p, int np, const float* u0, long long u0_bs, float* traj, int n, int include_init,
                           hipStream_t st) {

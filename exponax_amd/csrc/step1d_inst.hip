@@ -153,11 +153,25 @@ static RollFn pick_roll_kc(int kind) {
   }
 }
 
-// Multi-step kernels carrying 1 or 2 transforms per lane group; `fr`
-// selects the Fourier-resident variant (ETDRK2 only); `std_kc` says that the
-// plan's dealias cutoff is default_kmax(M).
+// Points per lane of the latency variant (nt = 3): half the usual, twice the
+// lanes per transform. With few trajectories a step is one wavefront's serial
+// chain of instruction issue, and half the points per lane is about half the
+// instructions, against one more LDS exchange per transform. 0: not built.
+constexpr int latency_pt(int m) { return m == 1024 ? 8 : (m >= 32 && m <= 512 && (m & (m - 1)) == 0) ? 4 : 0; }
+
+// Multi-step kernels carrying 1 or 2 transforms per lane group (nt = 1, 2),
+// or 1 on twice the lanes (nt = 3); `fr` selects the Fourier-resident variant
+// (ETDRK2 only); `std_kc` says that the plan's dealias cutoff is
+// default_kmax(M).
 RollFn EXMI_CAT(get_roll1d_, EXMI_M)(int kind, int order, int nt, int fr, int std_kc) {
   constexpr int M = EXMI_M, PT = EXMI_PT;
+  if (nt == 3) {
+    if constexpr (latency_pt(M) > 0) {
+      constexpr int LPT = latency_pt(M);
+      if (std_kc && order == 2) return fr ? pick_roll_kc<M, LPT, 1, true>(kind) : pick_roll_kc<M, LPT, 1, false>(kind);
+    }
+    return nullptr;
+  }
   if (std_kc && order == 2) {
     RollFn f = nullptr;
     if (nt == 1) f = fr ? pick_roll_kc<M, PT, 1, true>(kind) : pick_roll_kc<M, PT, 1, false>(kind);

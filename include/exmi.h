@@ -453,7 +453,9 @@ int exmi_plan_get_tables(const exmi_plan* plan, float* host_out, int64_t host_co
  * kernel; the per-step physical round trip), 1 or 2 = one multi-step launch
  * keeping 1 or 2 transforms per lane group on chip for all steps (the
  * Fourier-resident form where the plan has it, see
- * EXMI_FLAG_PHYSICAL_ROLLOUT). 2-D: 1 = the workgroup-resident kernel, 2 =
+ * EXMI_FLAG_PHYSICAL_ROLLOUT). 1-D, N = 64 .. 2048, ETDRK2, real L,
+ * convection and gradient norm with the 2/3 cutoff: 3 = as 1 on twice the
+ * lanes per transform (few trajectories). 2-D: 1 = the workgroup-resident kernel, 2 =
  * the spectrum-carrying launch chain, 3 = the same chain as one cooperative
  * launch (single-channel gradient norm and vorticity, N = 128 and 256, when
  * the whole grid fits the device; inside exmi_rollout_group with several
