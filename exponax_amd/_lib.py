@@ -155,26 +155,25 @@ def load_library(path: str = LIB_PATH):
 
 
 def lib():
-    """The library, after checking that a HIP device is present (once: the
-    answer is taken without a lock afterwards)."""
-    if _ready is not None:
-        return _ready
-    return _checked_library()
-
-
-_ready = None
-
-
-def _checked_library():
-    global _ready
+    """The library, after checking that a HIP device is present."""
     L = load_library()
+    _require_device()
+    return L
+
+
+_device_checked = False
+
+
+def _require_device():
+    global _device_checked
+    if _device_checked:
+        return
     import torch
 
     if not torch.cuda.is_available():
         raise ExmiError("exponax_amd needs a HIP device (torch.cuda.is_available() is False); "
                         "there is no CPU fallback")
-    _ready = L
-    return L
+    _device_checked = True
 
 
 def check(rc: int, what: str = "") -> None:
