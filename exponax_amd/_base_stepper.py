@@ -29,11 +29,14 @@ Plan options, set as attributes before the first call:
 """
 from __future__ import annotations
 
+import math
+
 import numpy as np
+import torch
 
 from . import _lib
 from . import spectral as sp
-from ._tensor import as_device_tensor, restore_like
+from ._tensor import as_device_tensor, as_float32, restore_like
 
 
 class BaseStepper:
@@ -120,34 +123,31 @@ class BaseStepper:
         return (self.num_channels,) + sp.wavenumber_shape(self.num_spatial_dims, self.num_points)
 
     def _split(self, t, trailing):
-        if tuple(t.shape[-len(trailing):]) != tuple(trailing):
-            raise ValueError(f"Expected shape (..., {', '.join(map(str, trailing))}), got {tuple(t.shape)}.")
-        lead = tuple(t.shape[:-len(trailing)])
-        return lead, int(np.prod(lead)) if lead else 1
+        shape = tuple(t.shape)
+        if shape[-len(trailing):] != trailing:
+            raise ValueError(f"Expected shape (..., {', '.join(map(str, trailing))}), got {shape}.")
+        lead = shape[:-len(trailing)]
+        return lead, int(math.prod(lead))
 
     def step(self, u):
         """fft -> ETDRK step -> ifft (``_base_stepper.py:201-220``) on one
         state or a batch with leading axes."""
-        import torch
-
         t, back = as_device_tensor(u)
         lead, B = self._split(t, self.state_shape)
-        x = t.contiguous().to(torch.float32)
+        x = as_float32(t)
         out = torch.empty_like(x)
-        n = int(np.prod(self.state_shape))
+        n = int(math.prod(self.state_shape))
         p = self.plan(B)
         _lib.check(_lib.lib().exmi_step(p.handle, x.data_ptr(), n, out.data_ptr(), n, _lib.stream_ptr()), "exmi_step")
         return restore_like(out, back)
 
     def step_fourier(self, u_hat):
         """``_base_stepper.py:222-239``."""
-        import torch
-
         t, back = as_device_tensor(u_hat)
         lead, B = self._split(t, self.spectral_shape)
         x = t.contiguous().to(torch.complex64)
         out = torch.empty_like(x)
-        n = int(np.prod(self.spectral_shape))
+        n = int(math.prod(self.spectral_shape))
         p = self.plan(B)
         _lib.check(_lib.lib().exmi_step_fourier(p.handle, x.data_ptr(), n, out.data_ptr(), n, _lib.stream_ptr()),
                    "exmi_step_fourier")
@@ -164,14 +164,12 @@ class BaseStepper:
     # ----------------------------------------------------- native rollouts
     def rollout_batch(self, u0, n: int, *, include_init: bool = False, use_graph: bool = True):
         """(..., C, N^D) -> (..., n[+1], C, N^D) in one captured graph."""
-        import torch
-
         t, back = as_device_tensor(u0)
         lead, B = self._split(t, self.state_shape)
-        x = t.contiguous().to(torch.float32)
+        x = as_float32(t)
         T = n + (1 if include_init else 0)
         out = torch.empty(lead + (T,) + self.state_shape, dtype=torch.float32, device=x.device)
-        sz = int(np.prod(self.state_shape))
+        sz = int(math.prod(self.state_shape))
         p = self.plan(B)
         _lib.check(_lib.lib().exmi_rollout(p.handle, x.data_ptr(), sz, out.data_ptr(), n, int(include_init),
                                            int(use_graph), _lib.stream_ptr()), "exmi_rollout")
@@ -183,15 +181,13 @@ class BaseStepper:
         time index whose state has a non-finite value or one above `bound`
         in magnitude (bound <= 0: non-finite only), -1 if none
         (exmi_rollout_checked)."""
-        import torch
-
         t, back = as_device_tensor(u0)
         lead, B = self._split(t, self.state_shape)
-        x = t.contiguous().to(torch.float32)
+        x = as_float32(t)
         T = n + (1 if include_init else 0)
         out = torch.empty(lead + (T,) + self.state_shape, dtype=torch.float32, device=x.device)
         fb = torch.empty(B, dtype=torch.int32, device=x.device)
-        sz = int(np.prod(self.state_shape))
+        sz = int(math.prod(self.state_shape))
         p = self.plan(B)
         _lib.check(_lib.lib().exmi_rollout_checked(p.handle, x.data_ptr(), sz, out.data_ptr(), n, int(include_init),
                                                    float(bound), fb.data_ptr(), _lib.stream_ptr()),
@@ -199,13 +195,11 @@ class BaseStepper:
         return restore_like(out, back), restore_like(fb.reshape(lead) if lead else fb[0], back)
 
     def repeat_batch(self, u0, n: int, *, use_graph: bool = True):
-        import torch
-
         t, back = as_device_tensor(u0)
         lead, B = self._split(t, self.state_shape)
-        x = t.contiguous().to(torch.float32)
+        x = as_float32(t)
         out = torch.empty_like(x)
-        sz = int(np.prod(self.state_shape))
+        sz = int(math.prod(self.state_shape))
         p = self.plan(B)
         _lib.check(_lib.lib().exmi_repeat(p.handle, x.data_ptr(), sz, out.data_ptr(), n, int(use_graph),
                                           _lib.stream_ptr()), "exmi_repeat")
@@ -215,8 +209,6 @@ class BaseStepper:
         """``repeat_batch`` of the contiguous float32 device batch ``x`` that
         also returns the states after ``every``, 2 ``every``, ... < n steps
         (exmi_repeat_checkpointed), for ``_repeat_vjp``."""
-        import torch
-
         _, B = self._split(x, self.state_shape)
         k = every if 0 < every < n else max(n, 1)
         out = torch.empty_like(x)
@@ -230,10 +222,8 @@ class BaseStepper:
     def _repeat_vjp(self, x, n: int, ckpt, g, every: int):
         """Gradient of ``repeat_batch`` from the checkpoints of its forward
         pass (exmi_repeat_vjp)."""
-        import torch
-
         _, B = self._split(x, self.state_shape)
-        g = g.contiguous().to(torch.float32)
+        g = as_float32(g)
         out = torch.empty_like(x)
         p = self.plan(B)
         _lib.check(_lib.lib().exmi_repeat_vjp(p.handle, x.data_ptr(), x.numel() // B, n, ckpt.data_ptr(),
@@ -245,17 +235,15 @@ class BaseStepper:
     def step_vjp(self, u, g):
         """(d step(u) / d u)^T g for one state or a batch (the reverse-mode
         derivative jax.vjp gives for ``_base_stepper.py:241-271``)."""
-        import torch
-
         t, back = as_device_tensor(u)
         gt, _ = as_device_tensor(g)
         lead, B = self._split(t, self.state_shape)
         if tuple(gt.shape) != tuple(t.shape):
             raise ValueError(f"cotangent shape {tuple(gt.shape)} != state shape {tuple(t.shape)}")
-        x = t.contiguous().to(torch.float32)
-        gx = gt.contiguous().to(torch.float32)
+        x = as_float32(t)
+        gx = as_float32(gt)
         out = torch.empty_like(x)
-        n = int(np.prod(self.state_shape))
+        n = int(math.prod(self.state_shape))
         p = self.plan(B)
         _lib.check(_lib.lib().exmi_step_vjp(p.handle, x.data_ptr(), n, gx.data_ptr(), n, out.data_ptr(), n,
                                             _lib.stream_ptr()), "exmi_step_vjp")
@@ -266,12 +254,10 @@ class BaseStepper:
         """Gradient through ``rollout(n, include_init)`` (cotangents g_traj of
         the trajectory) and/or through ``repeat(n)`` (cotangent g_final of the
         last state), recomputing segments of `checkpoint_every` steps."""
-        import torch
-
         t, back = as_device_tensor(u0)
         lead, B = self._split(t, self.state_shape)
-        x = t.contiguous().to(torch.float32)
-        sz = int(np.prod(self.state_shape))
+        x = as_float32(t)
+        sz = int(math.prod(self.state_shape))
         T = n + (1 if include_init else 0)
         gtp = gfp = None
         keep = []
@@ -279,14 +265,14 @@ class BaseStepper:
             gt, _ = as_device_tensor(g_traj)
             if tuple(gt.shape) != lead + (T,) + self.state_shape:
                 raise ValueError(f"g_traj shape {tuple(gt.shape)} != {lead + (T,) + self.state_shape}")
-            gt = gt.contiguous().to(torch.float32)
+            gt = as_float32(gt)
             keep.append(gt)
             gtp = gt.data_ptr()
         if g_final is not None:
             gf, _ = as_device_tensor(g_final)
             if tuple(gf.shape) != tuple(t.shape):
                 raise ValueError(f"g_final shape {tuple(gf.shape)} != state shape {tuple(t.shape)}")
-            gf = gf.contiguous().to(torch.float32)
+            gf = as_float32(gf)
             keep.append(gf)
             gfp = gf.data_ptr()
         out = torch.empty_like(x)
@@ -348,8 +334,6 @@ class _ScaledNonlinearFun:
         self._base.fill(desc)
 
     def __call__(self, u_hat):
-        import torch
-
         t, back = as_device_tensor(u_hat)
         if t.dim() < 1 or t.shape[0] != len(self.factors):
             raise ValueError(f"this ensemble's nonlinear function takes a batch of {len(self.factors)} spectra")
@@ -419,8 +403,6 @@ class Ensemble(BaseStepper):
     def _by_group(self, name, x, *args, **kw):
         """Run method `name` of every group on its members' states (the
         leading axis of x) and scatter the results back in member order."""
-        import torch
-
         t, back = as_device_tensor(x)
         if t.dim() < 1 or t.shape[0] != self.batch:
             raise ValueError(f"this ensemble advances exactly {self.batch} states, got {tuple(t.shape)}")

@@ -155,25 +155,26 @@ def load_library(path: str = LIB_PATH):
 
 
 def lib():
-    """The library, after checking that a HIP device is present."""
+    """The library, after checking that a HIP device is present (once: the
+    answer is taken without a lock afterwards)."""
+    if _ready is not None:
+        return _ready
+    return _checked_library()
+
+
+_ready = None
+
+
+def _checked_library():
+    global _ready
     L = load_library()
-    _require_device()
-    return L
-
-
-_device_checked = False
-
-
-def _require_device():
-    global _device_checked
-    if _device_checked:
-        return
     import torch
 
     if not torch.cuda.is_available():
         raise ExmiError("exponax_amd needs a HIP device (torch.cuda.is_available() is False); "
                         "there is no CPU fallback")
-    _device_checked = True
+    _ready = L
+    return L
 
 
 def check(rc: int, what: str = "") -> None:

@@ -4,20 +4,28 @@ in the caller's kind."""
 from __future__ import annotations
 
 import numpy as np
+import torch
+
+from . import _lib
+
+_TORCH = ("torch", None)
+
+
+def as_float32(t):
+    """``t`` as a contiguous float32 tensor, itself where it is one."""
+    if t.dtype is torch.float32 and t.is_contiguous():
+        return t
+    return t.contiguous().to(torch.float32)
 
 
 def as_device_tensor(x):
     """Return (CUDA tensor, restore-info). Raises ExmiError without a HIP
     device: the kernels are the only compute path."""
-    import torch
-
-    from . import _lib
-
     _lib.lib()
 
     if isinstance(x, torch.Tensor):
         if x.is_cuda:
-            return x, ("torch", None)
+            return x, _TORCH
         return x.cuda(), ("torch_cpu", None)
     if isinstance(x, np.ndarray) or np.isscalar(x):
         return torch.as_tensor(np.asarray(x)).cuda(), ("numpy", None)
@@ -30,6 +38,8 @@ def as_device_tensor(x):
 
 
 def restore_like(t, info):
+    if info is _TORCH:
+        return t
     kind, _ = info
     if kind == "torch":
         return t
