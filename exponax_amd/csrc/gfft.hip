@@ -49,7 +49,7 @@ __global__ void __launch_bounds__(GFFT_WG) gfft_kernel(GfftArgs a) {
   const int n = a.d.n, nz = n / 2 + 1, tid = threadIdx.x;
   const long long run0 = (long long)(REAL ? blockIdx.x : xcd_block()) * a.lpb;
   const int L = (int)(a.nrun - run0 < a.lpb ? a.nrun - run0 : a.lpb);
-  const int pitch = gfft_pitch(a.lpb);
+  const int pitch = REAL ? gfft_pitch(a.lpb) : gfft_pitch_by_point(n, a.lpb);
   cf* A = gfft_smem;
   cf* B = gfft_smem + n * pitch;
   // TWL: the twiddle table is staged in LDS (it fits beside the two line buffers)
@@ -235,7 +235,7 @@ hipError_t launch_gfft(const GfftCfg& c, int mode, const void* in, void* out, co
   }
   const long long grid = (a.nrun + c.lpb - 1) / c.lpb;
   if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
-  const size_t buf = sizeof(cf) * 2 * (size_t)c.n * gfft_pitch(c.lpb), fixed = 2 * sizeof(long long) * GFFT_MAX_LINES;
+  const size_t buf = sizeof(cf) * 2 * (size_t)c.n * (real ? gfft_pitch(c.lpb) : gfft_pitch_by_point(c.n, c.lpb)), fixed = 2 * sizeof(long long) * GFFT_MAX_LINES;
   size_t lds = buf + sizeof(cf) * (size_t)c.n;
   const bool twl = lds + fixed <= GFFT_LDS_MAX;
   if (!twl) lds = buf;

@@ -89,6 +89,11 @@ GfftDev gfft_dev(const GfftCfg& c, bool reversed = false);
 // side by side, with an odd pitch so that neither neighbouring lines nor the
 // passes' strided points share banks.
 __host__ __device__ __forceinline__ int gfft_pitch(int lines) { return lines | 1; }
+// The same where the lines are filled point by point, all lines of a point by
+// neighbouring threads: an odd n has odd radices only, whose strides spread an
+// even pitch over the banks as well, and the entry saved admits another
+// workgroup to the CU (four lines of n = 513: 37 KiB, four instead of three).
+__host__ __device__ __forceinline__ int gfft_pitch_by_point(int n, int lines) { return n & 1 ? lines : lines | 1; }
 // Workgroups are dealt to the 8 XCDs in turn, each with an L2 of its own;
 // logical block numbers that run through one XCD's workgroups first. A
 // strided axis is read and written in segments of a few lines (24 bytes at

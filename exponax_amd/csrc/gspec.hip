@@ -39,7 +39,7 @@ __global__ void __launch_bounds__(GFFT_WG) gfields_kernel(GFieldsArgs g) {
   const int n = g.d.n, tid = threadIdx.x;
   const long long run0 = (long long)xcd_block() * g.lpb;
   const int L = (int)(g.nrun - run0 < g.lpb ? g.nrun - run0 : g.lpb);
-  const int pitch = gfft_pitch(g.lpb);
+  const int pitch = gfft_pitch_by_point(n, g.lpb);
   cf* A = gspec_smem;
   cf* B = gspec_smem + n * pitch;
   const cf* T = TWL ? gspec_smem + 2 * n * pitch : g.tw;
@@ -94,7 +94,7 @@ hipError_t launch_gfields(const GfftCfg& c, const NL3DArgs& a, const cf* S, cf* 
   g.tw = tw;
   const long long grid = (g.nrun + c.lpb - 1) / c.lpb;
   if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
-  const size_t buf = sizeof(cf) * 2 * (size_t)c.n * gfft_pitch(c.lpb), fixed = 28 * GFFT_MAX_LINES;
+  const size_t buf = sizeof(cf) * 2 * (size_t)c.n * gfft_pitch_by_point(c.n, c.lpb), fixed = 28 * GFFT_MAX_LINES;
   size_t lds = buf + sizeof(cf) * (size_t)c.n;
   const bool twl = lds + fixed <= GFFT_LDS_MAX;
   if (!twl) lds = buf;
@@ -128,19 +128,25 @@ __global__ void __launch_bounds__(GFFT_WG) gprod_kernel(GProdArgs g) {
   const long long u0 = (long long)blockIdx.x * g.units;
   const int U = (int)(g.nunits - u0 < g.units ? g.nunits - u0 : g.units);
   const int LF = U * g.nft, LP = U * g.npt;
-  const int pf = gfft_pitch(g.units * g.nft), pp = gfft_pitch(g.units * g.npt);
+  const int pf = gfft_pitch_by_point(n, g.units * g.nft), pp = gfft_pitch_by_point(n, g.units * g.npt);
   const int half = n * (pf > pp ? pf : pp);
   cf* A = gspec_smem;
   cf* B = gspec_smem + half;
   const cf* T = TWL ? gspec_smem + 2 * half : g.tw;
   if constexpr (TWL)
     for (int i = tid; i < n; i += GFFT_WG) gspec_smem[2 * half + i] = g.tw[i];
-  const long long per = (g.rows + 1) / 2;  // units per trajectory
   const float rnz = 1.f / (float)nz, rU = 1.f / (float)U, rnf = 1.f / (float)g.nft, rnp = 1.f / (float)g.npt;
   const float rkk = 1.f / (float)g.kkeep;
-  // where line l of unit u starts: row 0, and whether it has a row 1
+  // where line l of unit u starts: row 0, and whether it has a row 1. The
+  // first unit's trajectory and row are divided out once; a unit further on
+  // is rarely past the trajectory's end.
+  const long long per = (g.rows + 1) / 2, tb = u0 / per, tq = u0 - tb * per;  // per: units per trajectory
   auto where = [&](int u, int l, int count, long long& at, bool& two) {
-    const long long unit = u0 + u, b = unit / per, q = unit - b * per;
+    long long b = tb, q = tq + u;
+    while (q >= per) {
+      q -= per;
+      ++b;
+    }
     at = (b * count + l) * g.a.Nr + 2 * q * nz;
     two = 2 * q + 1 < g.rows;
   };
@@ -192,7 +198,7 @@ __global__ void __launch_bounds__(GFFT_WG) gprod_kernel(GProdArgs g) {
 
 // LDS of one workgroup of `units` units, without and with the twiddle table.
 static size_t gprod_lds(int n, int nft, int npt, int units, bool tw) {
-  const int pf = gfft_pitch(units * nft), pp = gfft_pitch(units * npt);
+  const int pf = gfft_pitch_by_point(n, units * nft), pp = gfft_pitch_by_point(n, units * npt);
   return sizeof(cf) * ((size_t)2 * n * (pf > pp ? pf : pp) + (tw ? n : 0));
 }
 
@@ -209,12 +215,21 @@ hipError_t launch_gprod(const GfftCfg& c, const NL3DArgs& a, const cf* F, cf* P,
   g.nft = a.channels * a.nf;
   g.npt = a.channels * a.np;
   const int most = g.nft > g.npt ? g.nft : g.npt;
+  g.rows = a.dims == 3 ? (long long)a.nx * a.ny : a.ny;
+  g.nunits = a.ninst / a.channels * ((g.rows + 1) / 2);
   g.units = c.lpb / most;  // the tuned lines per workgroup
+  // Short lines leave most of a workgroup's lanes without a butterfly: at
+  // least about 1152 points to a workgroup while that leaves three workgroups
+  // to a CU (3-D Burgers, two of 12 fields, two units instead of one: 20 steps
+  // at 48^3 2266 -> 2090 us, 16 at 45^3 1751 -> 1585; four vorticity fields of
+  // 16 x 135^2, 1088 units, would lose 1015 -> 1047).
+  long long fill = 1152 / ((long long)most * c.n);
+  if (fill > g.nunits / 768) fill = g.nunits / 768;
+  if (fill > GFFT_MAX_LINES / most) fill = GFFT_MAX_LINES / most;
+  if (g.units < fill) g.units = (int)fill;
   if (g.units < 1) g.units = 1;
   while (g.units > 1 && gprod_lds(c.n, g.nft, g.npt, g.units, false) > GFFT_LDS_MAX) --g.units;
   g.kkeep = kkeep;
-  g.rows = a.dims == 3 ? (long long)a.nx * a.ny : a.ny;
-  g.nunits = a.ninst / a.channels * ((g.rows + 1) / 2);
   g.scale = scale;
   g.F = F;
   g.P = P;
@@ -276,7 +291,7 @@ __global__ void __launch_bounds__(GFFT_WG) gstage_kernel(GStageArgs g, Stage3DAr
   const int n = g.d.n, tid = threadIdx.x;
   const long long u0 = (long long)xcd_block() * g.units;
   const int U = (int)(g.nunits - u0 < g.units ? g.nunits - u0 : g.units);
-  const int L = U * g.npt, pitch = gfft_pitch(g.units * g.npt);
+  const int L = U * g.npt, pitch = gfft_pitch_by_point(n, g.units * g.npt);
   cf* A = gspec_smem;
   cf* B = gspec_smem + n * pitch;
   const cf* T = TWL ? gspec_smem + 2 * n * pitch : g.tw;
@@ -315,7 +330,7 @@ __global__ void __launch_bounds__(GFFT_WG) gstage_kernel(GStageArgs g, Stage3DAr
 }
 
 static size_t gstage_lds(int n, int npt, int units, bool tw) {
-  return sizeof(cf) * ((size_t)2 * n * gfft_pitch(units * npt) + (tw ? n : 0));
+  return sizeof(cf) * ((size_t)2 * n * gfft_pitch_by_point(n, units * npt) + (tw ? n : 0));
 }
 constexpr size_t GSTAGE_FIXED = 20 * GFFT_MAX_LINES;
 

@@ -76,11 +76,12 @@ def test_1d_per_member_tables_and_channels(device):
         assert torch.equal(got[i:i + 1], one)
 
 
-@pytest.mark.parametrize("N", [6, 33, 99, 810, 825])
+@pytest.mark.parametrize("N", [6, 33, 99, 810, 825, 1025])
 def test_2d_rows_with_products(device, N):
-    """Kolmogorov flow (four fields): 810 is the largest smooth size below
-    the row kernel's LDS limit (four 64 KiB line pairs), 825 runs the
-    separate passes; 33, 99 and 825 leave a last row alone."""
+    """Kolmogorov flow (four fields): 810 is the largest smooth even size below
+    the row kernel's LDS limit (64 KiB of line pairs), which odd sizes reach
+    above 1024: 1025 runs the separate passes; 33, 99, 825 and 1025 leave a
+    last row alone."""
     import torch
 
     print(f"[case] kolmogorov N={N}", flush=True)
