@@ -127,7 +127,7 @@ template <int N, int MODE>
 __global__ void __launch_bounds__(RowCfg<N>::WG) row2d_adj_kernel(Adj2DArgs aa) {
   __shared__ cf lds_x[RowLds<N>::X];
   __shared__ cf lds_t[RowLds<N>::TL];
-  row2d_adj_body<N, MODE, false>(aa, blockIdx.x, blockIdx.y, lds_x, lds_t);
+  row2d_adj_body<N, MODE, false>(aa, row_group<N>(), blockIdx.y, lds_x, lds_t);
 }
 
 template <int N, int MODE>

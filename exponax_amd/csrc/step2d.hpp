@@ -56,6 +56,9 @@
 #ifndef EXMI_ROW_R
 #define EXMI_ROW_R 16
 #endif
+#ifndef EXMI_ROW_R512
+#define EXMI_ROW_R512 4
+#endif
 #ifndef EXMI_COL_PT4_MAX
 #define EXMI_COL_PT4_MAX 128
 #endif
@@ -166,7 +169,14 @@ struct RowCfg {
   // shorter per-lane chain for these latency-bound sizes
   static constexpr int PT = N <= EXMI_ROW_PT4_MAX ? 4 : 8;
   static constexpr int T = M / PT;
-  static constexpr int R = EXMI_ROW_R;  // rows per workgroup
+  // Rows per workgroup. A row pass is a chain per workgroup (tile in, tile to
+  // rows, transform, per field), so the CU needs several workgroups whose
+  // chains interleave: at N = 512 sixteen rows are 70 KiB of LDS and 32
+  // workgroups per instance, one to a CU at 8 instances. Four rows (17 KiB)
+  // measured 2511 -> 2459 us of 40 Kolmogorov steps at 8 instances, 2171 ->
+  // 2091 of 20 at 16, 1027 -> 871 at 2; eight rows 2506, 2055, 934. Below 512
+  // the cooperative rollouts pair 16-row workgroups with the column groups.
+  static constexpr int R = N >= 512 ? EXMI_ROW_R512 : EXMI_ROW_R;
   static constexpr int WG = R * T;
   static constexpr int NY = M + 1;
   static constexpr int LD = R + 1;  // padded tile row
@@ -487,11 +497,21 @@ __device__ __forceinline__ void row2d_body(const Step2DArgs& a, int bx, int inst
   }
 }
 
+// The row group of this workgroup. Four rows are 32-byte segments of T and F:
+// the workgroups that share a cache line run on one XCD, so its L2 merges them
+// (workgroups are dealt to the 8 XCDs in turn).
+template <int N>
+__device__ __forceinline__ int row_group() {
+  constexpr int RG = N / RowCfg<N>::R;
+  if constexpr (RowCfg<N>::R < 16 && RG % 8 == 0) return (blockIdx.x & 7) * (RG / 8) + (blockIdx.x >> 3);
+  else return blockIdx.x;
+}
+
 template <int N, int MODE, int KIND>
 __global__ void __launch_bounds__(RowCfg<N>::WG) row2d_kernel(Step2DArgs a) {
   __shared__ cf lds_x[RowLds<N>::X];
   __shared__ cf lds_t[RowLds<N>::TL];
-  row2d_body<N, MODE, KIND, false>(a, blockIdx.x, blockIdx.y, lds_x, lds_t);
+  row2d_body<N, MODE, KIND, false>(a, row_group<N>(), blockIdx.y, lds_x, lds_t);
 }
 
 template <int N, int MODE, int KIND>
