@@ -2635,7 +2635,9 @@ static int effective_nt(const exmi_plan* p) {
     if (p->coop2d) return 3;
     return p->fr2d ? 2 : -1;
   }
-  // 1-D: the latency variant while it needs no more wavefronts than there are SIMDs
+  // 1-D: the latency variant while it needs no more wavefronts than there are
+  // SIMDs (us per 100 KS steps, usual / latency, N = 256: 1024 trajectories
+  // 336 / 287, 2048 378 / 327, 4096 403 / 410, 8192 510 / 723)
   if (p->roll[3] && (long long)p->d.batch * p->d.num_channels * (p->M / 4) <= 1024 * 64LL) return 3;
   return p->roll[2] ? 2 : (p->roll[1] ? 1 : -1);
 }
