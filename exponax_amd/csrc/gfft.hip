@@ -202,7 +202,8 @@ static const int k_gfft_cands[] = {8 * 100000 + 512,   8 * 100000 + 1024,
                                    100000000 + 10 * 100000 + 1024, 100000000 + 10 * 100000 + 2048,
                                    100000000 + 16 * 100000 + 512,  100000000 + 16 * 100000 + 1024,
                                    100000000 + 16 * 100000 + 2048, 100000000 + 16 * 100000 + 4096,
-                                   100000000 + 8 * 100000 + 1024,  100000000 + 8 * 100000 + 2048};
+                                   100000000 + 8 * 100000 + 1024,  100000000 + 8 * 100000 + 2048,
+                                   100000000 + 8 * 100000 + 256,   100000000 + 8 * 100000 + 768};
 int gfft_num_candidates() { return (int)(sizeof k_gfft_cands / sizeof k_gfft_cands[0]); }
 int gfft_candidate(int i) { return k_gfft_cands[i]; }
 int gfft_default_code() { return 100000000 + 8 * 100000 + 2048; }
