@@ -17,6 +17,7 @@ from __future__ import annotations
 import torch
 
 from ._base_stepper import BaseStepper
+from ._tensor import as_float32
 
 
 class _Step(torch.autograd.Function):
@@ -54,10 +55,9 @@ class _Repeat(torch.autograd.Function):
         # the checkpoints the backward starts its segments from are states
         # this pass goes through: kept here, the backward need not run it again
         ctx.keep = (ctx.needs_input_grad[0] and n > checkpoint_every > 0 and isinstance(stepper, BaseStepper)
-                    and getattr(stepper, "_groups", None) is None and u0.dtype == torch.float32
-                    and u0.is_contiguous())
+                    and getattr(stepper, "_groups", None) is None)
         if ctx.keep:
-            out, ckpt = stepper._repeat_checkpointed(u0.detach(), n, checkpoint_every)
+            out, ckpt = stepper._repeat_checkpointed(as_float32(u0.detach()), n, checkpoint_every)
             ctx.save_for_backward(u0, ckpt)
             return out
         ctx.save_for_backward(u0)
@@ -67,7 +67,7 @@ class _Repeat(torch.autograd.Function):
     def backward(ctx, g):
         if ctx.keep:
             u0, ckpt = ctx.saved_tensors
-            return ctx.stepper._repeat_vjp(u0.detach(), ctx.n, ckpt, g, ctx.k), None, None, None
+            return ctx.stepper._repeat_vjp(as_float32(u0.detach()), ctx.n, ckpt, g, ctx.k), None, None, None
         (u0,) = ctx.saved_tensors
         return ctx.stepper.rollout_vjp(u0.detach(), ctx.n, g_final=g.contiguous(), checkpoint_every=ctx.k), None, \
             None, None
@@ -92,6 +92,9 @@ def rollout(stepper, u0, n: int, *, include_init: bool = False, checkpoint_every
 
 
 def repeat(stepper, u0, n: int, *, checkpoint_every: int = 10):
-    """``exponax.repeat(stepper, n)(u0)``, differentiable in ``u0``."""
+    """``exponax.repeat(stepper, n)(u0)``, differentiable in ``u0``: the bits
+    of ``stepper.repeat_batch``. Where ``u0`` requires a gradient the states after
+    every ``checkpoint_every`` steps are kept with the graph until its backward
+    (ceil(n / checkpoint_every) - 1 batches of states)."""
     _check(u0)
     return _Repeat.apply(u0, stepper, n, checkpoint_every)

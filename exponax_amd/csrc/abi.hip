@@ -1337,12 +1337,16 @@ static hipError_t stages3d(exmi_plan* p, Stage3DArgs& sa, hipStream_t st, cf* em
   return e;
 }
 
-// 1-D plans of a runtime size that fit LDS (p->g1): n steps in one launch,
-// states to out + b * out_bs + t * out_ts (only the last, at out + b * out_bs,
-// with final_only); roundtrip: every step starts from the emitted float32
-// state, else the spectrum is carried.
+// The multi-step launches below write the states after every, 2 every, ...
+// steps and the last one (1: every state, n: the last one only) to out +
+// b * out_bs, one out_ts apart; the last one to last + b * out_bs instead
+// where that is given (next_written, written_at).
+
+// 1-D plans of a runtime size that fit LDS (p->g1): n steps in one launch;
+// roundtrip: every step starts from the emitted float32 state, else the
+// spectrum is carried.
 static int enqueue_g1d(exmi_plan* p, const float* u0, long long u0_bs, float* out, long long out_bs,
-                       long long out_ts, int n, int final_only, int roundtrip, hipStream_t st) {
+                       long long out_ts, int n, int every, float* last, int roundtrip, hipStream_t st) {
   G1dArgs g;
   fill_nl3d(p, g.nl);
   // alias-free quadratic products: u u_x and (1/2)(u^2)_x agree on every
@@ -1358,7 +1362,8 @@ static int enqueue_g1d(exmi_plan* p, const float* u0, long long u0_bs, float* ou
   g.lin_channels = p->d.lin_channels;
   g.e_im = p->cplx ? num_coefs(p->d.order) : -1;
   g.nsteps = n;
-  g.final_only = final_only;
+  g.every = every;
+  g.last = last;
   g.roundtrip = roundtrip;
   g.tables = p->tables;
   g.tw = p->tw_col.tw;
@@ -1379,7 +1384,7 @@ static int enqueue_g1d(exmi_plan* p, const float* u0, long long u0_bs, float* ou
 // evaluates N(u_hat) instead of a step (exmi_nonlinear).
 static int enqueue_step3d(exmi_plan* p, const float* u_in, long long ibs, float* u_out, long long obs,
                           hipStream_t st, bool in_f = false, bool out_f = false, bool nonlin_only = false) {
-  if (p->g1 && !in_f && !out_f && !nonlin_only) return enqueue_g1d(p, u_in, ibs, u_out, obs, 0, 1, 1, 0, st);
+  if (p->g1 && !in_f && !out_f && !nonlin_only) return enqueue_g1d(p, u_in, ibs, u_out, obs, 0, 1, 1, nullptr, 0, st);
   const int B = p->d.batch, C = p->d.num_channels;
   const long long sz = (long long)p->d.num_channels * p->n3;
   const long long szs = 2LL * p->d.num_channels * p->nr;  // floats of one spectrum
@@ -1440,11 +1445,9 @@ static int enqueue_step3d(exmi_plan* p, const float* u_in, long long ibs, float*
 // Multi-pass spectrum-carrying rollout (strategy 2): the initial states are
 // transformed once; each step advances the spectra (the stages of
 // enqueue_step3d, alternating the state between W3 and S3) and emits its
-// state with the inverse transform that leaves the spectrum in place. States
-// go to out + i * out_bs + t * out_ts (only the last, at out, with
-// final_only).
+// state with the inverse transform that leaves the spectrum in place.
 static int enqueue_md_carry(exmi_plan* p, const float* u0, long long u0_bs, float* out, long long out_bs,
-                            long long out_ts, int n, int final_only, hipStream_t st) {
+                            long long out_ts, int n, int every, float* last, hipStream_t st) {
   const int B = p->d.batch;
   const long long sz = (long long)p->d.num_channels * p->n3;
   hipError_t e = hipSuccess;
@@ -1474,12 +1477,13 @@ static int enqueue_md_carry(exmi_plan* p, const float* u0, long long u0_bs, floa
   sa.NC = p->NC3;
   sa.S1 = p->S13;
   sa.A = p->A3;
+  int slot = 0, next = next_written(0, every, n);
   for (int t = 0; t < n && e == hipSuccess; ++t) {
     if (p->d.order == 0) {
       e = launch_etdrk0_spec(cur, p->ninst, p->nr, p->d.num_channels, p->tables, p->ncoef, p->d.lin_batch,
                              p->d.lin_channels, -1, st);
     }
-    const bool emit = !(final_only && t < n - 1);
+    const bool emit = t + 1 == next;
     bool emitted = false;  // the last stage left the new state's x lines in K3
     if (p->d.order > 0) {
       sa.U0 = cur;
@@ -1491,7 +1495,8 @@ static int enqueue_md_carry(exmi_plan* p, const float* u0, long long u0_bs, floa
       nxt = t2;
     }
     if (e != hipSuccess || !emit) continue;
-    float* dst = final_only ? out : out + (long long)t * out_ts;
+    float* dst = written_at(out, out_ts, slot++, last, t + 1 == n);
+    next = next_written(next, every, n);
     if (emitted) {
       const int N = p->d.num_points;
       e = launch_yz_inverse3d(N, p->K3, dst, p->ninst * N, p->tw_col.tw, p->tw.rt(),
@@ -2141,7 +2146,7 @@ int exmi_plan_get_tables(const exmi_plan* p, float* host_out, int64_t host_count
 }
 
 static int enqueue_roll(exmi_plan* p, int nt, const float* u0, long long u0_bs, float* out, long long out_bs,
-                        long long out_ts, int n, int final_only, hipStream_t st, int* first_bad = nullptr,
+                        long long out_ts, int n, int every, float* last, hipStream_t st, int* first_bad = nullptr,
                         float bound = 0.f, int bad_offset = 0);
 
 static int run_step(exmi_plan* p, const void* in, long long in_bs, int in_f, void* out, long long out_bs, int out_f,
@@ -2159,7 +2164,7 @@ static int run_step(exmi_plan* p, const void* in, long long in_bs, int in_f, voi
     if (nonlin_only || in_f || out_f)
       return fail(EXMI_ERR_UNSUPPORTED, "channel-coupled reaction plans step physical states only");
     const long long sz = (long long)p->d.num_channels * p->d.num_points;
-    return enqueue_roll(p, 1, (const float*)in, in_bs, (float*)out, out_bs, sz, 1, 0, st);
+    return enqueue_roll(p, 1, (const float*)in, in_bs, (float*)out, out_bs, sz, 1, 1, nullptr, st);
   }
   hipError_t e = nonlin_only ? p->nonlin(a, st) : p->step(a, st);
   if (e != hipSuccess) return fail(EXMI_ERR_HIP, "step launch failed: %s", hipGetErrorString(e));
@@ -2225,7 +2230,7 @@ static hipError_t copy_batch(const float* src, long long ss, float* dst, long lo
 }
 
 static int enqueue_roll(exmi_plan* p, int nt, const float* u0, long long u0_bs, float* out, long long out_bs,
-                        long long out_ts, int n, int final_only, hipStream_t st, int* first_bad,
+                        long long out_ts, int n, int every, float* last, hipStream_t st, int* first_bad,
                         float bound, int bad_offset) {
   Roll1DArgs ra;
   fill_args(p, &ra.s);
@@ -2238,15 +2243,15 @@ static int enqueue_roll(exmi_plan* p, int nt, const float* u0, long long u0_bs, 
   ra.traj_bstride = out_bs;
   ra.traj_tstride = out_ts;
   ra.nsteps = n;
-  ra.final_only = final_only;
+  ra.every = every;
+  ra.last = last;
   hipError_t e = p->roll[nt](ra, st);
   return e == hipSuccess ? EXMI_OK : fail(EXMI_ERR_HIP, "rollout launch failed: %s", hipGetErrorString(e));
 }
 
-// 2-D workgroup-resident rollout: one launch for all n steps, instance i's
-// states to out + i * out_bs + t * out_ts (only the last with final_only).
+// 2-D workgroup-resident rollout: one launch for all n steps.
 static int enqueue_roll2d(exmi_plan* p, const float* u0, long long u0_bs, float* out, long long out_bs,
-                          long long out_ts, int n, int final_only, hipStream_t st) {
+                          long long out_ts, int n, int every, float* last, hipStream_t st) {
   Roll2DArgs ra;
   fill_args2d(p, &ra.s);
   ra.u0 = u0;
@@ -2255,7 +2260,8 @@ static int enqueue_roll2d(exmi_plan* p, const float* u0, long long u0_bs, float*
   ra.traj_bstride = out_bs;
   ra.traj_tstride = out_ts;
   ra.nsteps = n;
-  ra.final_only = final_only;
+  ra.every = every;
+  ra.last = last;
   ra.ninst = p->ninst;
   const hipError_t e = p->roll2d(ra, st);
   return e == hipSuccess ? EXMI_OK : fail(EXMI_ERR_HIP, "2-D rollout launch failed: %s", hipGetErrorString(e));
@@ -2264,10 +2270,8 @@ static int enqueue_roll2d(exmi_plan* p, const float* u0, long long u0_bs, float*
 // 2-D spectrum-resident launch chain: RA CA once, then per step
 // RB|RCB CB RB CCA, and a final RC. RCB emits the previous step's state
 // while forming the products; CCA keeps S' as the next S0 with its fields.
-// States go to out + i * out_bs + t * out_ts (only the last, at out, with
-// final_only).
 static int enqueue_chain_fr2d(exmi_plan* p, const float* u0, long long u0_bs, float* out, long long out_bs,
-                              long long out_ts, int n, int final_only, hipStream_t st) {
+                              long long out_ts, int n, int every, float* last, hipStream_t st) {
   Step2DArgs a;
   fill_args2d(p, &a);
   a.u_in = u0;
@@ -2277,11 +2281,13 @@ static int enqueue_chain_fr2d(exmi_plan* p, const float* u0, long long u0_bs, fl
   const int B = p->ninst;
   hipError_t e = p->row2d[ROW_RA](a, B, st);
   if (e == hipSuccess) e = p->col2d[COL_CA](a, B, st);
+  int slot = 0, next = next_written(0, every, n);
   for (int t = 0; t < n && e == hipSuccess; ++t) {
-    if (t == 0 || final_only) {
+    if (t != next) {
       e = p->row2d[ROW_RB](a, B, st);
     } else {
-      a.u_out = out + (long long)(t - 1) * out_ts;
+      a.u_out = out + (long long)slot++ * out_ts;
+      next = next_written(next, every, n);
       e = p->row2d[ROW_RCB](a, B, st);
     }
     if (e == hipSuccess) e = p->col2d[COL_CB](a, B, st);
@@ -2290,16 +2296,15 @@ static int enqueue_chain_fr2d(exmi_plan* p, const float* u0, long long u0_bs, fl
     if (e == hipSuccess) e = p->col2d[COL_CCA](a, B, st);
   }
   if (e == hipSuccess) {
-    a.u_out = final_only ? out : out + (long long)(n - 1) * out_ts;
+    a.u_out = written_at(out, out_ts, slot, last, true);
     e = p->row2d[ROW_RC](a, B, st);
   }
   return e == hipSuccess ? EXMI_OK : fail(EXMI_ERR_HIP, "2-D rollout launch failed: %s", hipGetErrorString(e));
 }
 
-// The chain as one cooperative launch for all n steps (states as in
-// enqueue_chain_fr2d).
+// The chain as one cooperative launch for all n steps.
 static int enqueue_coop2d(exmi_plan* p, const float* u0, long long u0_bs, float* out, long long out_bs,
-                          long long out_ts, int n, int final_only, hipStream_t st, float* G = nullptr,
+                          long long out_ts, int n, int every, float* last, hipStream_t st, float* G = nullptr,
                           long long G_tstride = 0) {
   Coop2DArgs ca;
   memset(&ca, 0, sizeof ca);
@@ -2312,7 +2317,8 @@ static int enqueue_coop2d(exmi_plan* p, const float* u0, long long u0_bs, float*
   ca.traj_bstride = out_bs;
   ca.traj_tstride = out_ts;
   ca.nsteps = n;
-  ca.final_only = final_only;
+  ca.every = every;
+  ca.last = last;
   ca.ninst = p->ninst;
   ca.sync = p->coop_sync;
   ca.spin_limit = p->coop_spin;
@@ -2335,8 +2341,8 @@ static int enqueue_rollout_nt(exmi_plan* p, int nt, const float* u0, long long u
   if (n == 0) return EXMI_OK;
   if (p->md) {
     if (p->g1)
-      return enqueue_g1d(p, u0, u0_bs, traj + off * sz, tstride, sz, n, 0, !(nt == 2 && p->md_carry), st);
-    if (nt == 2 && p->md_carry) return enqueue_md_carry(p, u0, u0_bs, traj + off * sz, tstride, sz, n, 0, st);
+      return enqueue_g1d(p, u0, u0_bs, traj + off * sz, tstride, sz, n, 1, nullptr, !(nt == 2 && p->md_carry), st);
+    if (nt == 2 && p->md_carry) return enqueue_md_carry(p, u0, u0_bs, traj + off * sz, tstride, sz, n, 1, nullptr, st);
     for (int t = 0; t < n; ++t) {
       const float* in = (t == 0 && !include_init) ? u0 : traj + (long long)(t - 1 + off) * sz;
       const long long ibs = (t == 0 && !include_init) ? u0_bs : tstride;
@@ -2346,9 +2352,9 @@ static int enqueue_rollout_nt(exmi_plan* p, int nt, const float* u0, long long u
     return EXMI_OK;
   }
   if (p->ndim == 2) {
-    if (nt == 1 && p->roll2d) return enqueue_roll2d(p, u0, u0_bs, traj + off * sz, tstride, sz, n, 0, st);
-    if (nt == 2 && p->fr2d) return enqueue_chain_fr2d(p, u0, u0_bs, traj + off * sz, tstride, sz, n, 0, st);
-    if (nt == 3 && p->coop2d) return enqueue_coop2d(p, u0, u0_bs, traj + off * sz, tstride, sz, n, 0, st);
+    if (nt == 1 && p->roll2d) return enqueue_roll2d(p, u0, u0_bs, traj + off * sz, tstride, sz, n, 1, nullptr, st);
+    if (nt == 2 && p->fr2d) return enqueue_chain_fr2d(p, u0, u0_bs, traj + off * sz, tstride, sz, n, 1, nullptr, st);
+    if (nt == 3 && p->coop2d) return enqueue_coop2d(p, u0, u0_bs, traj + off * sz, tstride, sz, n, 1, nullptr, st);
     for (int t = 0; t < n; ++t) {
       int rc = enqueue_step2d(p, u0, u0_bs, traj + (long long)(t + off) * sz, tstride, t > 0, t < n - 1, st);
       if (rc) return rc;
@@ -2358,7 +2364,7 @@ static int enqueue_rollout_nt(exmi_plan* p, int nt, const float* u0, long long u
   // nt = -1 on a plan that chose the Fourier-resident kernels itself: the
   // per-step launches (the literal physical round trip) stay available
   if (p->fourier_resident && (nt == 0 || (nt < 0 && !p->fr_auto))) nt = p->roll[2] ? 2 : 1;
-  if (nt > 0 && p->roll[nt]) return enqueue_roll(p, nt, u0, u0_bs, traj + off * sz, tstride, sz, n, 0, st);
+  if (nt > 0 && p->roll[nt]) return enqueue_roll(p, nt, u0, u0_bs, traj + off * sz, tstride, sz, n, 1, nullptr, st);
   for (int t = 0; t < n; ++t) {
     const float* in = (t == 0 && !include_init) ? u0 : traj + (long long)(t - 1 + off) * sz;
     const long long ibs = (t == 0 && !include_init) ? u0_bs : tstride;
@@ -2658,45 +2664,60 @@ static int effective_nt(const exmi_plan* p) {
 // one segment).
 static int vjp_segment(int n, int every) { return every > 0 && every < n ? every : (n > 0 ? n : 1); }
 
-static int enq_repeat_cb(exmi_plan* p, const void* a, const void* b, long long s, int n, int, hipStream_t st) {
-  const float* u0 = (const float*)a;
-  float* out = (float*)b;
-  const long long sz = state_size(p);
+// n steps from u0 (batch stride s) to out, whose states after K, 2 K, ... < n
+// steps also go to ckpt (none with K >= n), each a contiguous batch: of every
+// strategy the rollout whose last state alone is written without them, so the
+// result does not depend on K.
+static int enqueue_repeat(exmi_plan* p, const float* u0, long long s, float* out, int n, int K, float* ckpt,
+                          hipStream_t st) {
+  const long long sz = state_size(p), bsz = (long long)p->d.batch * sz;
+  float* const last = K < n ? out : nullptr;
+  float* const first = K < n ? ckpt : out;
   if (n == 0) {
     hipError_t e = copy_batch(u0, s, out, sz, sz, p->d.batch, st);
     return e == hipSuccess ? EXMI_OK : fail(EXMI_ERR_HIP, "copy failed: %s", hipGetErrorString(e));
   }
+  // per-step launches: where the state after step t + 1 goes (to out where it is not asked for)
+  auto state = [&](int t) { return K < n && t + 1 < n && (t + 1) % K == 0 ? ckpt + ((t + 1) / K - 1) * bsz : out; };
   if (p->md) {
     const bool carry = effective_nt(p) == 2 && p->md_carry;
-    if (p->g1) return enqueue_g1d(p, u0, s, out, sz, 0, n, 1, !carry, st);
-    if (carry) return enqueue_md_carry(p, u0, s, out, sz, 0, n, 1, st);
+    if (p->g1) return enqueue_g1d(p, u0, s, first, sz, bsz, n, K, last, !carry, st);
+    if (carry) return enqueue_md_carry(p, u0, s, first, sz, bsz, n, K, last, st);
+    const float* in = u0;
     for (int t = 0; t < n; ++t) {
-      int rc = enqueue_step3d(p, t == 0 ? u0 : out, t == 0 ? s : sz, out, sz, st);
+      float* o = state(t);
+      int rc = enqueue_step3d(p, in, t == 0 ? s : sz, o, sz, st);
       if (rc) return rc;
+      in = o;
     }
     return EXMI_OK;
   }
   if (p->ndim == 2) {
     const int nt2 = effective_nt(p);
-    if (nt2 == 1 && p->roll2d) return enqueue_roll2d(p, u0, s, out, sz, 0, n, 1, st);
-    if (nt2 == 2 && p->fr2d) return enqueue_chain_fr2d(p, u0, s, out, sz, 0, n, 1, st);
-    if (nt2 == 3 && p->coop2d) return enqueue_coop2d(p, u0, s, out, sz, 0, n, 1, st);
+    if (nt2 == 1 && p->roll2d) return enqueue_roll2d(p, u0, s, first, sz, bsz, n, K, last, st);
+    if (nt2 == 2 && p->fr2d) return enqueue_chain_fr2d(p, u0, s, first, sz, bsz, n, K, last, st);
+    if (nt2 == 3 && p->coop2d) return enqueue_coop2d(p, u0, s, first, sz, bsz, n, K, last, st);
     for (int t = 0; t < n; ++t) {
-      int rc = enqueue_step2d(p, u0, s, out, sz, t > 0, t < n - 1, st);
+      int rc = enqueue_step2d(p, u0, s, state(t), sz, t > 0, t < n - 1, st);
       if (rc) return rc;
     }
     return EXMI_OK;
   }
   const int nt = effective_nt(p);
-  if (nt > 0 && p->roll[nt]) return enqueue_roll(p, nt, u0, s, out, sz, 0, n, 1, st);
-  for (int t = 0; t < n; ++t) {
-    const float* in = t == 0 ? u0 : (((n - t) % 2 == 0) ? out : p->work);
-    const long long ibs = t == 0 ? s : sz;
-    float* o = ((n - 1 - t) % 2 == 0) ? out : p->work;
-    int rc = run_step(p, in, ibs, 0, o, sz, 0, 0, st);
+  if (nt > 0 && p->roll[nt]) return enqueue_roll(p, nt, u0, s, first, sz, bsz, n, K, last, st);
+  const float* in = u0;
+  for (int t = 0; t < n; ++t) {  // in turn to out and the workspace, the last one to out
+    float* o = state(t);
+    if (o == out && (n - 1 - t) % 2) o = p->work;
+    int rc = run_step(p, in, t == 0 ? s : sz, 0, o, sz, 0, 0, st);
     if (rc) return rc;
+    in = o;
   }
   return EXMI_OK;
+}
+
+static int enq_repeat_cb(exmi_plan* p, const void* a, const void* b, long long s, int n, int, hipStream_t st) {
+  return enqueue_repeat(p, (const float*)a, s, (float*)b, n, n, nullptr, st);
 }
 
 int exmi_rollout(exmi_plan* p, const float* u0, int64_t u0_bs, float* traj, int32_t n, int32_t include_init,
@@ -2773,7 +2794,7 @@ int exmi_rollout_checked(exmi_plan* p, const float* u0, int64_t u0_bs, float* tr
     }
     hipLaunchKernelGGL(exmi_fill_int_kernel, dim3(small_grid(B)), dim3(256), 0, st, (int*)first_bad, B, INT_MAX);
     HIP_TRY(hipGetLastError());
-    int rc = enqueue_roll(p, nt, u0, u0_bs, traj + off * sz, tstride, sz, n, 0, st, (int*)first_bad, bnd, off);
+    int rc = enqueue_roll(p, nt, u0, u0_bs, traj + off * sz, tstride, sz, n, 1, nullptr, st, (int*)first_bad, bnd, off);
     if (rc) return rc;
     hipLaunchKernelGGL(exmi_bad_finalize_kernel, dim3(small_grid(B)), dim3(256), 0, st, (int*)first_bad, B);
     HIP_TRY(hipGetLastError());
@@ -2939,18 +2960,11 @@ int exmi_repeat_checkpointed(exmi_plan* p, const float* u0, int64_t u0_bs, float
   if (n < 0) return fail(EXMI_ERR_INVALID, "n_steps must be >= 0");
   const int K = vjp_segment(n, every), nseg = n > 0 ? (n + K - 1) / K : 1;
   if (nseg > 1 && !ckpt) return fail(EXMI_ERR_INVALID, "null argument");
-  if (K > 1) {
+  if (n > 1) {
     int rc = ensure_work(p);
     if (rc) return rc;
   }
-  const long long sz = state_size(p), bsz = (long long)p->d.batch * sz;
-  for (int s = 0; s < nseg; ++s) {
-    const float* in = s == 0 ? u0 : ckpt + (s - 1) * bsz;
-    float* out = s == nseg - 1 ? u_out : ckpt + s * bsz;
-    int rc = enq_repeat_cb(p, in, out, s == 0 ? u0_bs : sz, n - s * K < K ? n - s * K : K, 0, (hipStream_t)stream);
-    if (rc) return rc;
-  }
-  return EXMI_OK;
+  return enqueue_repeat(p, u0, u0_bs, u_out, n, nseg > 1 ? K : n, ckpt, (hipStream_t)stream);
 }
 
 }  // extern "C"
@@ -3528,7 +3542,7 @@ static int rollout_vjp(exmi_plan* p, const float* u0, int64_t u0_bs, int32_t n, 
         // the segment's len steps as one cooperative launch that keeps the
         // gradient fields of every step (its states are not needed; the last
         // one lands in seg), then the transposed steps from those fields
-        rc = enqueue_coop2d(p, from, fbs, seg, sz, 0, len, 1, st, p->Gseg, gblk);
+        rc = enqueue_coop2d(p, from, fbs, seg, sz, 0, len, len, nullptr, st, p->Gseg, gblk);
         if (rc) return rc;
       } else {
         rc = enqueue_rollout_nt(p, effective_nt(p), from, fbs, seg, len - 1, 1, st);

@@ -46,7 +46,8 @@ struct Coop2DArgs {
   long long traj_bstride;  // floats between instances
   long long traj_tstride;  // floats between consecutive outputs of one instance
   int nsteps;
-  int final_only;          // 1: write only the last state, at traj
+  int every;               // written: the states after every, 2 every, ... steps and the last one
+  float* last;             // where the last one goes, or null: in its turn
   int ninst;
   unsigned* sync;          // arrival counter of instance i at sync[64 i] (zero at launch);
                            // sync[64 ninst]: failure word (nonzero: a barrier gave up)
@@ -119,16 +120,18 @@ __global__ void __launch_bounds__(CoopCfg<N>::WG) coop2d_kernel(Coop2DArgs ca) {
   cf* rt = lds + RowLds<N>::X;
   const bool row = g < CC::RG;
   const int n = ca.nsteps;
-  int next_out = 0;  // first state this workgroup's rows have not been written to yet
+  int slot = 0;  // first output this workgroup's rows have not been written to yet
+  int next = next_written(0, ca.every, n);
   // after a barrier gave up: this workgroup's rows of every state not yet
   // written become NaN, so no stale data passes for a result
   auto give_up = [&]() {
     if (!row) return;
     const int x0 = g * RowCfg<N>::R;
-    const int t0 = ca.final_only ? 0 : next_out, t1 = ca.final_only ? 1 : n;
-    for (int t = t0; t < t1; ++t) {
-      float* o = ca.traj + (long long)inst * ca.traj_bstride + (long long)t * ca.traj_tstride + (long long)x0 * N;
+    for (int t = next;; t = next_written(t, ca.every, n)) {
+      float* o = written_at(ca.traj, ca.traj_tstride, slot++, ca.last, t == n) + (long long)inst * ca.traj_bstride +
+                 (long long)x0 * N;
       for (int i = threadIdx.x; i < RowCfg<N>::R * N; i += CC::WG) o[i] = __builtin_nanf("");
+      if (t == n) break;
     }
   };
 
@@ -140,12 +143,13 @@ __global__ void __launch_bounds__(CoopCfg<N>::WG) coop2d_kernel(Coop2DArgs ca) {
     a.Gout = ca.G ? ca.G + (long long)t * ca.G_tstride : nullptr;
     a.gstage = 0;
     if (row) {
-      if (t == 0 || ca.final_only) {
+      if (t != next) {
         row2d_body<N, ROW_RB, KIND, true>(a, g, inst, rx, rt);
       } else {
-        a.u_out = ca.traj + (long long)(t - 1) * ca.traj_tstride;
+        a.u_out = ca.traj + (long long)slot * ca.traj_tstride;
         row2d_body<N, ROW_RCB, KIND, true>(a, g, inst, rx, rt);
-        next_out = t;
+        ++slot;
+        next = next_written(next, ca.every, n);
       }
     }
     if (!meet()) return give_up();
@@ -159,7 +163,7 @@ __global__ void __launch_bounds__(CoopCfg<N>::WG) coop2d_kernel(Coop2DArgs ca) {
     if (!meet()) return give_up();
   }
   if (row) {
-    a.u_out = ca.final_only ? ca.traj : ca.traj + (long long)(n - 1) * ca.traj_tstride;
+    a.u_out = written_at(ca.traj, ca.traj_tstride, slot, ca.last, true);
     row2d_body<N, ROW_RC, KIND, true>(a, g, inst, rx, rt);
   }
 }

@@ -52,4 +52,16 @@ __host__ __device__ inline int num_coefs_c(int order, bool cplx) {
   return num_coefs(order) + (cplx ? (order >= 3 ? 2 : 1) : 0);
 }
 
+// Which states of a rollout of n steps are written: those after every,
+// 2 every, ... steps and the one after the last step (every = 1: all of them,
+// n: only the last). next_written: the step after which the next one is
+// written, the last having been after step t (0: none yet). written_at: where
+// number `slot` goes: one tstride after the one before, the last one to `last`
+// unless that is null.
+__host__ __device__ __forceinline__ int next_written(int t, int every, int n) { return n - t > every ? t + every : n; }
+__host__ __device__ __forceinline__ float* written_at(float* base, long long tstride, int slot, float* last,
+                                                      bool is_last) {
+  return is_last && last ? last : base + (long long)slot * tstride;
+}
+
 }  // namespace exmi

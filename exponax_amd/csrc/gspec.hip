@@ -435,6 +435,7 @@ __global__ void __launch_bounds__(G1D_WG_MAX) g1d_kernel(G1dArgs g) {
   }
   __syncthreads();
   forward(A, B);
+  int slot = 0, next = next_written(0, g.every, g.nsteps);
   for (int t = 0; t < g.nsteps; ++t) {
     if (g.order == 0) {
       for (int idx = tid; idx < S1N; idx += nthr) {
@@ -487,7 +488,7 @@ __global__ void __launch_bounds__(G1D_WG_MAX) g1d_kernel(G1dArgs g) {
       }
       __syncthreads();
     }
-    const bool emit = !g.final_only || t == g.nsteps - 1;
+    const bool emit = t + 1 == next;
     if (emit || g.roundtrip) {
       for (int idx = tid; idx < S1N; idx += nthr) {
         const int c = fdiv(idx, rnz), k = idx - c * nz;
@@ -500,7 +501,7 @@ __global__ void __launch_bounds__(G1D_WG_MAX) g1d_kernel(G1dArgs g) {
       __syncthreads();
       cf* Z = gfft_run<true, RMAX>(A, B, T, g.d, C, pitch, tid, nthr);
       cf* O = Z == A ? B : A;
-      float* out = g.out + b * g.out_bs + (g.final_only ? 0 : t * g.out_ts);
+      float* out = written_at(g.out, g.out_ts, slot, g.last, t + 1 == g.nsteps) + b * g.out_bs;
       for (int idx = tid; idx < C * n; idx += nthr) {
         const int c = fdiv(idx, rn), pt = idx - c * n;
         const float v = scale * Z[pt * pitch + c].re;
@@ -508,6 +509,10 @@ __global__ void __launch_bounds__(G1D_WG_MAX) g1d_kernel(G1dArgs g) {
         if (g.roundtrip) O[pt * pitch + c] = cf{v, 0.f};
       }
       __syncthreads();
+      if (emit) {
+        ++slot;
+        next = next_written(next, g.every, g.nsteps);
+      }
       if (g.roundtrip) {
         if (t < g.nsteps - 1) forward(O, Z);
         continue;
@@ -558,7 +563,7 @@ __global__ void __launch_bounds__(G1D_WG_MAX) g1s_kernel(G1dArgs g) {
   extern __shared__ cf sm[];
   const int tid = threadIdx.x, nthr = blockDim.x;
   const int n = g.nl.N, nz = g.nl.NZ, np = g.d.npass, kmax = g.nl.kmax, order = g.order, nsteps = g.nsteps;
-  const int final_only = g.final_only, e_im = g.e_im;
+  const int every = g.every, e_im = g.e_im;
   const bool grad = g.nl.kind == NL_GRADNORM, poly = g.nl.kind == NL_POLY;
   const float kscale = g.nl.kscale, scale = 1.f / (float)n;
   const GfftPass i0 = g.d.p[0], i1 = g.d.p[1], i2 = g.d.p[2], i3 = g.d.p[3];
@@ -579,8 +584,10 @@ __global__ void __launch_bounds__(G1D_WG_MAX) g1s_kernel(G1dArgs g) {
       sm[a + i] = cf{u0[i], 0.f};
     }
   }
-  float* const out = g.out + traj * g.out_bs;
-  const long long out_ts = final_only ? 0 : g.out_ts;
+  float* at = g.out + traj * g.out_bs;  // where the next written state goes
+  float* const last = g.last ? g.last + traj * g.out_bs : nullptr;
+  const long long out_ts = g.out_ts;
+  int next = next_written(0, every, nsteps);
   __syncthreads();
   // one inner pass of L lines side by side, LDS to LDS
   auto pass = [&](auto inv, const GfftPass p, int L) __attribute__((always_inline)) {
@@ -611,9 +618,13 @@ __global__ void __launch_bounds__(G1D_WG_MAX) g1s_kernel(G1dArgs g) {
   __syncthreads();
   for (int t = 0; t <= nsteps; ++t) {
     // t == nsteps: only the last state's emission
-    const bool emit = t > 0 && (!final_only || t == nsteps), step = t < nsteps;
+    const bool emit = t == next, step = t < nsteps;
     const int stages = step ? order : 1;
-    float* const dst = out + (t - 1) * out_ts;
+    float* const dst = step || !last ? at : last;
+    if (emit) {
+      at += out_ts;
+      next = next_written(next, every, nsteps);
+    }
     for (int i = 0; i < stages; ++i) {
       const int iX = i == 0 ? iU : iS;
       const int L = (i == 0 && emit && step) ? 2 : 1;

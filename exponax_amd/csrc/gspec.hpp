@@ -31,13 +31,15 @@ struct G1dArgs {
   NL3DArgs nl;
   GfftDev d, df;  // the inverse's passes (and the forward's); df the same in reverse order
   int order, ncoef, lin_batch, lin_channels, e_im;
-  int nsteps, final_only;
+  int nsteps;
+  int every;    // written: the states after every, 2 every, ... steps and the last one
+  float* last;  // where the last one goes, or null: in its turn
   int roundtrip;  // 1: every step transforms the emitted state forward again, 0: the spectrum is carried
   const float* tables;
   const cf* tw;
   const float* u0;
   long long u0_bs;
-  float* out;  // state of trajectory b after step t at out + b * out_bs + t * out_ts (final_only: the last one at out + b * out_bs)
+  float* out;  // the written states of trajectory b at out + b * out_bs (last + b * out_bs), one out_ts apart
   long long out_bs, out_ts;
 };
 bool g1d_fits(int N, int channels, int nf, int np, int order, int lin_channels, int ncoef);

@@ -52,7 +52,8 @@ struct Roll2DArgs {
   long long traj_bstride;  // floats between instances
   long long traj_tstride;  // floats between consecutive outputs of one instance
   int nsteps;
-  int final_only;          // 1: write only the last state
+  int every;               // written: the states after every, 2 every, ... steps and the last one
+  float* last;             // where the last one goes, or null: in its turn
   int ninst;
 };
 
@@ -228,8 +229,8 @@ __global__ void __launch_bounds__(R2Cfg<N>::WG) roll2d_kernel(Roll2DArgs ra) {
   };
 
   // ---- inverse transform of the state (2 u_hat) -> physical rows, written
-  // to the trajectory at output slot t
-  auto emit = [&](const cf* S, long long t) {
+  // to `to`
+  auto emit = [&](const cf* S, float* to) {
     cf v[1][PT];
 #pragma unroll
     for (int s = 0; s < PT; ++s) {
@@ -261,8 +262,7 @@ __global__ void __launch_bounds__(R2Cfg<N>::WG) roll2d_kernel(Roll2DArgs ra) {
       trr.load(jr, RealTables{a.tw_row, a.fw_row});
       irfft<M, PT, 1>(z, nyq, lnr, ldr, trr);
     }
-    float2* out = reinterpret_cast<float2*>(ra.traj + (long long)inst * ra.traj_bstride + t * ra.traj_tstride +
-                                            (long long)xr * N);
+    float2* out = reinterpret_cast<float2*>(to + (long long)inst * ra.traj_bstride + (long long)xr * N);
 #pragma unroll
     for (int s = 0; s < PT; ++s) out[jr + TR * s] = make_float2(z[0][s].re * rn2, z[0][s].im * rn2);
     __syncthreads();
@@ -310,6 +310,7 @@ __global__ void __launch_bounds__(R2Cfg<N>::WG) roll2d_kernel(Roll2DArgs ra) {
   auto n_outside = [&](int s) -> cf {
     return (KIND == NL_VORT && a.inj_mode == ky && jc + TC * s == 0) ? cf{2.f * a.inj_value, 0.f} : cf{0.f, 0.f};
   };
+  int slot = 0, next = next_written(0, ra.every, ra.nsteps);
   for (int step = 0; step < ra.nsteps; ++step) {
     {
       cf N0[PT];
@@ -334,8 +335,10 @@ __global__ void __launch_bounds__(R2Cfg<N>::WG) roll2d_kernel(Roll2DArgs ra) {
       const cf n0 = kept_col ? n0s[ky * N + jc + TC * s] : n_outside(s);
       S[s] = S[s] + coef(2, ky, s) * (N1[s] - n0);
     }
-    if (!ra.final_only) emit(S, step);
-    else if (step == ra.nsteps - 1) emit(S, 0);
+    if (step + 1 == next) {
+      emit(S, written_at(ra.traj, ra.traj_tstride, slot++, ra.last, step + 1 == ra.nsteps));
+      next = next_written(next, ra.every, ra.nsteps);
+    }
   }
 }
 

@@ -283,12 +283,13 @@ int exmi_step_vjp(exmi_plan* plan, const float* u_in, int64_t in_bstride, const 
 int exmi_rollout_vjp(exmi_plan* plan, const float* u0, int64_t u0_bstride, int32_t n_steps, int32_t include_init,
                      const float* g_traj, const float* g_final, float* g_u0, int32_t checkpoint_every, void* stream);
 
-/* exmi_repeat that also keeps what its gradient starts from: with K =
- * checkpoint_every (one segment when K <= 0 or K >= n_steps) the states after
- * K, 2 K, ... < n_steps steps go to ckpt, (ceil(n/K) - 1, B, C, N^D)
- * contiguous. exmi_repeat_vjp with the same n_steps, checkpoint_every and ckpt
- * is exmi_rollout_vjp(..., g_final, ...) without its forward pass. ckpt may be
- * NULL where it holds nothing. Not captured into a graph. */
+/* exmi_repeat (the same bits in u_out) that also keeps what its gradient
+ * starts from: with K = checkpoint_every (one segment when K <= 0 or K >=
+ * n_steps) the states after K, 2 K, ... < n_steps steps go to ckpt,
+ * (ceil(n/K) - 1, B, C, N^D) contiguous, the caller's to hold until the
+ * gradient is taken. exmi_repeat_vjp with the same n_steps, checkpoint_every
+ * and ckpt is exmi_rollout_vjp(..., g_final, ...) without its forward pass.
+ * ckpt may be NULL where it holds nothing. Not captured into a graph. */
 int exmi_repeat_checkpointed(exmi_plan* plan, const float* u0, int64_t u0_bstride, float* u_out, float* ckpt,
                              int32_t n_steps, int32_t checkpoint_every, void* stream);
 int exmi_repeat_vjp(exmi_plan* plan, const float* u0, int64_t u0_bstride, int32_t n_steps, const float* ckpt,
