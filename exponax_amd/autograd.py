@@ -50,13 +50,11 @@ class _Rollout(torch.autograd.Function):
 
 class _Repeat(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, u0, stepper, n, checkpoint_every):
-        ctx.stepper, ctx.n, ctx.k = stepper, n, checkpoint_every
+    def forward(ctx, u0, stepper, n, checkpoint_every, keep):
+        ctx.stepper, ctx.n, ctx.k, ctx.keep = stepper, n, checkpoint_every, keep
         # the checkpoints the backward starts its segments from are states
         # this pass goes through: kept here, the backward need not run it again
-        ctx.keep = (ctx.needs_input_grad[0] and n > checkpoint_every > 0 and isinstance(stepper, BaseStepper)
-                    and getattr(stepper, "_groups", None) is None)
-        if ctx.keep:
+        if keep:
             out, ckpt = stepper._repeat_checkpointed(as_float32(u0.detach()), n, checkpoint_every)
             ctx.save_for_backward(u0, ckpt)
             return out
@@ -67,10 +65,11 @@ class _Repeat(torch.autograd.Function):
     def backward(ctx, g):
         if ctx.keep:
             u0, ckpt = ctx.saved_tensors
-            return ctx.stepper._repeat_vjp(as_float32(u0.detach()), ctx.n, ckpt, g, ctx.k), None, None, None
+            return ctx.stepper._repeat_vjp(as_float32(u0.detach()), ctx.n, ckpt, g, ctx.k), None, None, None, \
+                None
         (u0,) = ctx.saved_tensors
         return ctx.stepper.rollout_vjp(u0.detach(), ctx.n, g_final=g.contiguous(), checkpoint_every=ctx.k), None, \
-            None, None
+            None, None, None
 
 
 def _check(u):
@@ -93,8 +92,15 @@ def rollout(stepper, u0, n: int, *, include_init: bool = False, checkpoint_every
 
 def repeat(stepper, u0, n: int, *, checkpoint_every: int = 10):
     """``exponax.repeat(stepper, n)(u0)``, differentiable in ``u0``: the bits
-    of ``stepper.repeat_batch``. Where ``u0`` requires a gradient the states after
+    of ``stepper.repeat_batch``. Where a gradient can follow, the states after
     every ``checkpoint_every`` steps are kept with the graph until its backward
     (ceil(n / checkpoint_every) - 1 batches of states)."""
     _check(u0)
-    return _Repeat.apply(u0, stepper, n, checkpoint_every)
+    keep = torch.is_grad_enabled() and u0.requires_grad and _own_repeat(stepper) and 0 < (checkpoint_every or 0) < n
+    return _Repeat.apply(u0, stepper, n, checkpoint_every, keep)
+
+
+def _own_repeat(stepper):
+    """Whether the stepper's repeat is the library's, on one plan (an ensemble
+    of several groups has a plan for each)."""
+    return isinstance(stepper, BaseStepper) and getattr(stepper, "_groups", None) is None

@@ -63,3 +63,22 @@ def test_kept_checkpoints_give_the_gradient(device, name, n, every):
             (again,) = torch.autograd.grad(y, x, g)
             assert torch.equal(gx, again)
             assert float((gx - want).norm() / want.norm()) <= 2e-5, nt
+
+
+def test_only_a_graph_keeps_checkpoints(device, monkeypatch):
+    """Nothing is kept where no gradient can follow, although the input asks
+    for one."""
+    import torch
+
+    st = S.KuramotoSivashinskyConservative(1, 30.0, 64, 0.05)
+    x = torch.tensor(ics(2, 1, 1.0, 64, 3, seed=5)[0], device=device, requires_grad=True)
+    ref = st.repeat_batch(x.detach(), 6)
+    kept = []
+    monkeypatch.setattr(type(st), "_repeat_checkpointed",
+                        lambda *a, _f=type(st)._repeat_checkpointed: kept.append(1) or _f(*a))
+    with torch.no_grad():
+        assert torch.equal(ex.autograd.repeat(st, x, 6, checkpoint_every=2), ref)
+    assert torch.equal(ex.autograd.repeat(st, x.detach(), 6, checkpoint_every=2), ref)
+    assert not kept
+    ex.autograd.repeat(st, x, 6, checkpoint_every=2)
+    assert kept
