@@ -16,7 +16,7 @@ from __future__ import annotations
 
 import torch
 
-from ._base_stepper import BaseStepper
+from ._base_stepper import BaseStepper, Ensemble
 from ._tensor import as_float32
 
 
@@ -103,4 +103,6 @@ def repeat(stepper, u0, n: int, *, checkpoint_every: int = 10):
 def _own_repeat(stepper):
     """Whether the stepper's repeat is the library's, on one plan (an ensemble
     of several groups has a plan for each)."""
-    return isinstance(stepper, BaseStepper) and getattr(stepper, "_groups", None) is None
+    return (isinstance(stepper, BaseStepper) and getattr(stepper, "_groups", None) is None
+            and type(stepper).repeat_batch in (BaseStepper.repeat_batch, Ensemble.repeat_batch)
+            and type(stepper).rollout_vjp is BaseStepper.rollout_vjp)

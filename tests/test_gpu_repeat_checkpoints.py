@@ -82,3 +82,25 @@ def test_only_a_graph_keeps_checkpoints(device, monkeypatch):
     assert not kept
     ex.autograd.repeat(st, x, 6, checkpoint_every=2)
     assert kept
+
+
+def test_a_steppers_own_repeat_is_called(device):
+    """A stepper that repeats or differentiates in its own way keeps doing so."""
+    import torch
+
+    class Mine(S.KuramotoSivashinskyConservative):
+        def repeat_batch(self, u0, n, **kw):
+            return 2.0 * super().repeat_batch(u0, n, **kw)
+
+    class Scaled(S.KuramotoSivashinskyConservative):
+        def rollout_vjp(self, *a, **kw):
+            return 2.0 * super().rollout_vjp(*a, **kw)
+
+    u0 = torch.tensor(ics(2, 1, 1.0, 64, 3, seed=5)[0], device=device)
+    plain = S.KuramotoSivashinskyConservative(1, 30.0, 64, 0.05)
+    x = u0.clone().requires_grad_(True)
+    assert torch.equal(ex.autograd.repeat(Mine(1, 30.0, 64, 0.05), x, 6, checkpoint_every=2),
+                       2.0 * plain.repeat_batch(u0, 6))
+    (got,) = torch.autograd.grad(ex.autograd.repeat(Scaled(1, 30.0, 64, 0.05), x, 6, checkpoint_every=2).sum(), x)
+    want = 2.0 * plain.rollout_vjp(u0, 6, g_final=torch.ones_like(u0), checkpoint_every=2)
+    assert torch.equal(got, want)
