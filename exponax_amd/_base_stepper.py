@@ -210,20 +210,27 @@ class BaseStepper:
         also returns the states after ``every``, 2 ``every``, ... < n steps
         (exmi_repeat_checkpointed), for ``_repeat_vjp``."""
         _, B = self._split(x, self.state_shape)
-        k = every if 0 < every < n else max(n, 1)
         out = torch.empty_like(x)
-        ckpt = torch.empty((max(-(-n // k), 1) - 1,) + tuple(x.shape), dtype=torch.float32, device=x.device)
+        ckpt = torch.empty(self._checkpoint_shape(x, n, every), dtype=torch.float32, device=x.device)
         p = self.plan(B)
         _lib.check(_lib.lib().exmi_repeat_checkpointed(p.handle, x.data_ptr(), x.numel() // B, out.data_ptr(),
                                                        ckpt.data_ptr(), n, int(every), _lib.stream_ptr()),
                    "exmi_repeat_checkpointed")
         return out, ckpt
 
+    def _checkpoint_shape(self, x, n: int, every: int):
+        k = every if 0 < every < n else max(n, 1)
+        return (max(-(-n // k), 1) - 1,) + tuple(x.shape)
+
     def _repeat_vjp(self, x, n: int, ckpt, g, every: int):
         """Gradient of ``repeat_batch`` from the checkpoints of its forward
         pass (exmi_repeat_vjp)."""
+        # saved tensors come back in whatever form their hooks leave them
+        x, g, ckpt = (as_float32(as_device_tensor(t)[0]) for t in (x, g, ckpt))
         _, B = self._split(x, self.state_shape)
-        g = as_float32(g)
+        if tuple(g.shape) != tuple(x.shape) or tuple(ckpt.shape) != self._checkpoint_shape(x, n, every):
+            raise ValueError(f"cotangent shape {tuple(g.shape)} or checkpoints' {tuple(ckpt.shape)} do not belong to "
+                             f"{n} steps from states of shape {tuple(x.shape)}")
         out = torch.empty_like(x)
         p = self.plan(B)
         _lib.check(_lib.lib().exmi_repeat_vjp(p.handle, x.data_ptr(), x.numel() // B, n, ckpt.data_ptr(),

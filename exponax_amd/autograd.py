@@ -65,8 +65,7 @@ class _Repeat(torch.autograd.Function):
     def backward(ctx, g):
         if ctx.keep:
             u0, ckpt = ctx.saved_tensors
-            return ctx.stepper._repeat_vjp(as_float32(u0.detach()), ctx.n, ckpt, g, ctx.k), None, None, None, \
-                None
+            return ctx.stepper._repeat_vjp(u0.detach(), ctx.n, ckpt, g, ctx.k), None, None, None, None
         (u0,) = ctx.saved_tensors
         return ctx.stepper.rollout_vjp(u0.detach(), ctx.n, g_final=g.contiguous(), checkpoint_every=ctx.k), None, \
             None, None, None

@@ -1,7 +1,7 @@
 """autograd.repeat keeps its checkpoints in the forward pass: the gradient
 equals the one whose backward forms them itself (rollout_vjp), for every kind
-of plan the repeat has, with a ragged last segment, one segment and strided
-inputs. The final state is repeat_batch's, bit for bit."""
+of plan the repeat has, with a ragged last segment, one segment, strided inputs
+and saved-tensor hooks. The final state is repeat_batch's, bit for bit."""
 import numpy as np
 import pytest
 
@@ -104,3 +104,26 @@ def test_a_steppers_own_repeat_is_called(device):
     (got,) = torch.autograd.grad(ex.autograd.repeat(Scaled(1, 30.0, 64, 0.05), x, 6, checkpoint_every=2).sum(), x)
     want = 2.0 * plain.rollout_vjp(u0, 6, g_final=torch.ones_like(u0), checkpoint_every=2)
     assert torch.equal(got, want)
+
+
+def test_saved_tensor_hooks(device):
+    """The checkpoints may leave the device between forward and backward; what
+    comes back is looked at before a kernel reads it."""
+    import torch
+
+    st = S.KuramotoSivashinskyConservative(1, 30.0, 64, 0.05)
+    x = torch.tensor(ics(2, 1, 1.0, 64, 3, seed=5)[0], device=device, requires_grad=True)
+    y = ex.autograd.repeat(st, x, 6, checkpoint_every=2)
+    (want,) = torch.autograd.grad(y.sum(), x)
+    hooks = {"cpu": (lambda t: t.cpu(), lambda t: t),
+             "strided": (lambda t: t, lambda t: torch.stack([t, t], dim=-1)[..., 0]),
+             "double": (lambda t: t.double(), lambda t: t)}
+    for name, (pack, unpack) in hooks.items():
+        with torch.autograd.graph.saved_tensors_hooks(pack, unpack):
+            y = ex.autograd.repeat(st, x, 6, checkpoint_every=2)
+        (got,) = torch.autograd.grad(y.sum(), x)
+        assert torch.equal(got, want), name
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: t[:1]):
+        y = ex.autograd.repeat(st, x, 6, checkpoint_every=2)
+    with pytest.raises(ValueError):
+        torch.autograd.grad(y.sum(), x)
