@@ -13,15 +13,17 @@
 // direct-sum pass, so every n factors.
 //
 // What bounds it: LDS traffic and instruction issue, not memory (four fields
-// of eight 513^2 grids along y: 90 MB in and out). Real lines run two per
-// complex transform where they are neighbouring rows of one field; divisions
-// by runtime sizes are float multiplications; the lines of a workgroup share
-// their twiddle reads and lie side by side at an odd pitch.
+// of eight 513^2 grids along y: 67 MB in and out, 45 MB of it inside the
+// cutoff). Real lines run two per complex transform where they are neighbouring
+// rows of one field; divisions by runtime sizes are float multiplications, and
+// 64-bit ones are made once per line; the lines of a workgroup share their
+// twiddle reads and lie side by side at an odd pitch.
 // Measured (eight 513^2 fields, one transform along one axis): forward lines
-// 15 us, inverse lines 13 us, r2c 18 us, c2r 15 us, against 33, 33, 42 and
-// 43 us with one real line per transform, R^2 complex products per radix-R
-// butterfly and integer divisions; a prime pass of 199 points (N = 597, one
-// step of 100 trajectories) 60 us per step against 185 us with direct sums.
+// 14 us, inverse lines 13 us, r2c 14 us, c2r 12 us (16 and 15 us with a row's
+// start divided out at every point), against 33, 33, 42 and 43 us with one real
+// line per transform, R^2 complex products per radix-R butterfly and integer
+// divisions; a prime pass of 199 points (N = 597, one step of 100 trajectories)
+// 60 us per step against 185 us with direct sums.
 #include <cstdio>
 
 #include "gfft.hpp"
@@ -43,6 +45,7 @@ template <int MODE, int RMAX, bool TWL>
 __global__ void __launch_bounds__(GFFT_WG) gfft_kernel(GfftArgs a) {
   extern __shared__ cf gfft_smem[];
   __shared__ long long b0[GFFT_MAX_LINES], b1[GFFT_MAX_LINES];
+  __shared__ int two[GFFT_MAX_LINES];
   constexpr bool INV = MODE == GFFT_INV || MODE == GFFT_C2R;
   constexpr bool REAL = MODE == GFFT_R2C || MODE == GFFT_C2R;
   const int n = a.d.n, nz = n / 2 + 1, tid = threadIdx.x;
@@ -55,13 +58,17 @@ __global__ void __launch_bounds__(GFFT_WG) gfft_kernel(GfftArgs a) {
   const cf* T = TWL ? gfft_smem + 2 * n * pitch : a.tw;
   if constexpr (TWL)
     for (int i = tid; i < n; i += GFFT_WG) gfft_smem[2 * n * pitch + i] = a.tw[i];
-  // where each line starts: C2C b0; real lines: the row numbers (b1 < 0: one row)
+  // where each line starts: C2C b0; real lines: its first row in the real
+  // array b0 and in the complex one b1, and whether the row behind it is the
+  // line's second (one of the same field, so right behind it in both arrays)
   if (tid < L) {
     const long long run = run0 + tid;
     if constexpr (REAL) {
       const long long per = (a.g.rows + 1) / 2, f = run / per, q = run - f * per;
-      b0[tid] = f * a.g.rows + 2 * q;
-      b1[tid] = 2 * q + 1 < a.g.rows ? b0[tid] + 1 : -1;
+      const long long row = f * a.g.rows + 2 * q;
+      b0[tid] = a.g.rpg > 0 ? (row / a.g.rpg) * a.g.gstride + (row % a.g.rpg) * n : row * n;
+      b1[tid] = row * nz;
+      two[tid] = 2 * q + 1 < a.g.rows;
     } else {
       const int mk = gfft_midkeep(a.g.midn, a.g.cut);
       const long long r = run / a.g.kkeep, o = r / mk;
@@ -70,24 +77,21 @@ __global__ void __launch_bounds__(GFFT_WG) gfft_kernel(GfftArgs a) {
   }
   __syncthreads();
   const float rL = 1.f / (float)L, rn = a.d.rn, rnz = 1.f / (float)nz;
-  auto real_at = [&](long long row) {
-    return a.g.rpg > 0 ? (row / a.g.rpg) * a.g.gstride + (row % a.g.rpg) * n : row * n;
-  };
   // load: consecutive threads read consecutive addresses (along the line for
   // contiguous lines, across neighbouring lines for a strided axis)
   if constexpr (MODE == GFFT_R2C) {
     const float* in = static_cast<const float*>(a.in);
     for (int idx = tid; idx < L * n; idx += GFFT_WG) {
       const int ll = fdiv(idx, rn), pt = idx - ll * n;
-      cf v = cf{in[real_at(b0[ll]) + pt], 0.f};
-      if (b1[ll] >= 0) v.im = in[real_at(b1[ll]) + pt];
-      A[pt * pitch + ll] = v;
+      const float* x = in + b0[ll] + pt;
+      A[pt * pitch + ll] = cf{x[0], two[ll] ? x[n] : 0.f};
     }
   } else if constexpr (MODE == GFFT_C2R) {
     const cf* in = static_cast<const cf*>(a.in);
     for (int idx = tid; idx < L * nz; idx += GFFT_WG) {
       const int ll = fdiv(idx, rnz), k = idx - ll * nz;
-      cf p = in[b0[ll] * nz + k], q = b1[ll] >= 0 ? in[b1[ll] * nz + k] : cf{0.f, 0.f};
+      const cf* x = in + b1[ll] + k;
+      cf p = x[0], q = two[ll] ? x[nz] : cf{0.f, 0.f};
       const bool self = k == 0 || 2 * k == n;
       if (self) p.im = q.im = 0.f;
       A[k * pitch + ll] = cf{p.re - q.im, p.im + q.re};
@@ -109,13 +113,14 @@ __global__ void __launch_bounds__(GFFT_WG) gfft_kernel(GfftArgs a) {
     for (int idx = tid; idx < L * nz; idx += GFFT_WG) {
       const int ll = fdiv(idx, rnz), k = idx - ll * nz;
       const cf zk = Z[k * pitch + ll];
-      if (b1[ll] < 0) {
-        out[b0[ll] * nz + k] = zk;
+      cf* x = out + b1[ll] + k;
+      if (!two[ll]) {
+        x[0] = zk;
       } else {
         cf p, q;
         unpack_pair(zk, Z[(k == 0 ? 0 : n - k) * pitch + ll], p, q);
-        out[b0[ll] * nz + k] = p;
-        out[b1[ll] * nz + k] = q;
+        x[0] = p;
+        x[nz] = q;
       }
     }
   } else if constexpr (MODE == GFFT_C2R) {
@@ -123,8 +128,9 @@ __global__ void __launch_bounds__(GFFT_WG) gfft_kernel(GfftArgs a) {
     for (int idx = tid; idx < L * n; idx += GFFT_WG) {
       const int ll = fdiv(idx, rn), pt = idx - ll * n;
       const cf v = Z[pt * pitch + ll];
-      out[real_at(b0[ll]) + pt] = a.scale * v.re;
-      if (b1[ll] >= 0) out[real_at(b1[ll]) + pt] = a.scale * v.im;
+      float* x = out + b0[ll] + pt;
+      x[0] = a.scale * v.re;
+      if (two[ll]) x[n] = a.scale * v.im;
     }
   } else {
     cf* out = static_cast<cf*>(a.out);
@@ -249,7 +255,8 @@ hipError_t launch_gfft(const GfftCfg& c, int mode, const void* in, void* out, co
   }
   const long long grid = (a.nrun + c.lpb - 1) / c.lpb;
   if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
-  const size_t buf = sizeof(cf) * 2 * (size_t)c.n * (real ? gfft_pitch(c.lpb) : gfft_pitch_by_point(c.n, c.lpb)), fixed = 2 * sizeof(long long) * GFFT_MAX_LINES;
+  const size_t buf = sizeof(cf) * 2 * (size_t)c.n * (real ? gfft_pitch(c.lpb) : gfft_pitch_by_point(c.n, c.lpb));
+  const size_t fixed = 20 * GFFT_MAX_LINES;
   size_t lds = buf + sizeof(cf) * (size_t)c.n;
   const bool twl = lds + fixed <= GFFT_LDS_MAX;
   if (!twl) lds = buf;
