@@ -2399,7 +2399,7 @@ static std::string tune_key(const exmi_plan* p) {
   }
   char key[256];
   snprintf(key, sizeof key, "%s|D%d|N%d|C%d|B%d|k%d|o%d|lb%d|fr%d", arch, p->ndim, p->d.num_points,
-           p->d.num_channels, p->d.batch, p->kind, p->d.order, p->d.lin_batch,
+           p->d.num_channels, p->d.batch, p->md ? p->kind3 : p->kind, p->d.order, p->d.lin_batch,
            p->fourier_resident ? (p->fr_auto ? 2 : 1) : 0);
   return key;
 }
@@ -2435,16 +2435,27 @@ static void tune_store(const exmi_plan* p) {
   }
 }
 
-// Runtime-size transforms: the radices (largest pass max_radix) and the
-// lines per workgroup are timed at plan creation on a forward and an
-// inverse transform of the plan's own batch, and the fastest kept; with
-// EXMI_TUNE_CACHE the choice is looked up and stored like the rollout
-// strategies ("<arch>|gfft|D|N|count <code>").
+// Runtime-size transforms: the radices (largest pass max_radix) and the lines
+// per workgroup are timed at plan creation and the fastest kept. Timed: a step
+// of the plan, whose fused passes do most of the work and want fewer or more
+// lines per workgroup than a bare transform does (KS 2-D, 16 x 100^2: 1007 ->
+// 945 us of 20 steps), up to 4M points; in 1-D, without a nonlinear term and
+// for more points a forward and an inverse transform of up to 4M points.
+static bool tunes_step(const exmi_plan* p) {
+  return p->ndim >= 2 && p->d.order > 0 && p->ninst * p->n3 <= (1LL << 22);
+}
+
+// With EXMI_TUNE_CACHE the choice is looked up and stored like the rollout
+// strategies, under what it was timed on: a transform depends on D, N and the
+// number of fields ("<arch>|v2|gfft|D|N|I <code>"), a step on everything that
+// tune_key holds ("<arch>|v2|gstep|D|N|C|B|k|o|lb|fr <code>": a tile of two
+// fields is not one of four). v2: entries of libraries that timed transforms
+// only, on other kernels, are not taken.
 static std::string gfft_tune_key(const exmi_plan* p) {
-  std::string k = tune_key(p);
+  const std::string k = tune_key(p), arch = k.substr(0, k.find('|'));
+  if (tunes_step(p)) return arch + "|v2|gstep" + k.substr(arch.size());
   char key[256];
-  snprintf(key, sizeof key, "%s|gfft|D%d|N%d|I%d", k.substr(0, k.find('|')).c_str(), p->ndim, p->d.num_points,
-           p->ninst);
+  snprintf(key, sizeof key, "%s|v2|gfft|D%d|N%d|I%d", arch.c_str(), p->ndim, p->d.num_points, p->ninst);
   return key;
 }
 
@@ -2483,11 +2494,8 @@ static int tune_gfft(exmi_plan* p) {
       return EXMI_OK;
     }
   }
-  // Timed: a step of the plan, whose fused passes do most of the work and
-  // want fewer or more lines per workgroup than a bare transform does (KS 2-D,
-  // 16 x 100^2: 1007 -> 938 us of 20 steps), up to ~4M points; else transforms
-  // of about as many points. In the plan's own buffers, on zeros.
-  const bool whole = p->ndim >= 2 && p->d.order > 0 && p->ninst * p->n3 <= (1LL << 22);
+  // in the plan's own buffers, on zeros
+  const bool whole = tunes_step(p);
   long long I = (1LL << 22) / p->n3;
   if (I < 1) I = 1;
   if (I > p->ninst) I = p->ninst;

@@ -480,7 +480,9 @@ int exmi_plan_set_rollout_strategy(exmi_plan* plan, int32_t strategy);
  * and the lines one workgroup holds in LDS. exmi_plan_create times a set of
  * candidates on the plan's batch and keeps the fastest (with
  * EXMI_TUNE_CACHE set, it looks the choice up first and stores a new one,
- * keyed by GPU architecture, D, N and the number of fields).
+ * keyed by what was timed: GPU architecture, D, N and the number of fields
+ * for bare transforms, the plan's shape and equation as for the rollout
+ * strategies for a step).
  * exmi_plan_fft_config writes [code, source, lines per workgroup, passes,
  * radix_1 .. radix_passes] into info (up to len entries) and returns the
  * entry count, 0 for plans on the fused kernels; code = reg * 100000000 +
