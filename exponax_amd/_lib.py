@@ -243,7 +243,8 @@ class Plan:
         kernels): code = reg * 100000000 + max_radix * 100000 + points per
         workgroup (reg 1: radices 9..17 and 19 as register butterflies), where it
         came from (default / timed / cache / set), lines per workgroup and
-        the pass radices."""
+        the pass radices. 1-D plans whose steps run as one launch use other
+        radices there until another code is set (include/exmi.h)."""
         buf = (C.c_int32 * 32)()
         n = self._lib.exmi_plan_fft_config(self._h, buf, 32)
         check(min(n, 0), "exmi_plan_fft_config")

@@ -433,7 +433,7 @@ struct exmi_plan {
   GfftCfg gcfg;          // runtime-size transforms: radices and lines per workgroup
   int gcode = 0;         // their knobs, encoded (autotuned at plan creation)
   int g1 = 0;            // 1-D runtime size: whole rollouts in one launch (gspec.hip)
-  GfftCfg g1cfg;         // its radices (short chains of small butterflies)
+  GfftCfg g1cfg;         // its radices (short chains of small butterflies), until a code is set
   int gtuned = 0;        // 0: default knobs, 1: timed at plan creation, 2: from the tuning cache, 3: set
   // multi-pass adjoint: stage states, cotangents and the nonlinear VJP's
   // cotangent fields / products (allocated on first use)
@@ -1372,7 +1372,7 @@ static int enqueue_g1d(exmi_plan* p, const float* u0, long long u0_bs, float* ou
   g.out = out;
   g.out_bs = out_bs;
   g.out_ts = out_ts;
-  const hipError_t e = launch_g1d(p->gtuned == 3 ? p->gcfg : p->g1cfg, g, st);
+  const hipError_t e = launch_g1d(p->g1cfg, g, st);
   return e == hipSuccess ? EXMI_OK : fail(EXMI_ERR_HIP, "1-D rollout launch failed: %s", hipGetErrorString(e));
 }
 
@@ -2107,6 +2107,9 @@ int exmi_plan_set_fft_config(exmi_plan* p, int32_t code) {
   GfftCfg c;
   if (!gfft_cfg_from_code(p->d.num_points, code, &c))
     return fail(EXMI_ERR_INVALID, "transform knobs %d: max_radix * 100000 + points_per_workgroup expected", code);
+  // the one launch of 1-D steps has radices of its own: the code in use,
+  // given back, leaves them alone
+  if (code != p->gcode) p->g1cfg = c;
   p->gcfg = c;
   p->gcode = code;
   p->gtuned = 3;

@@ -491,6 +491,10 @@ int exmi_plan_set_rollout_strategy(exmi_plan* plan, int32_t strategy);
  * such passes as direct sums); source 0 default, 1 timed, 2 tuning cache,
  * 3 set.
  * exmi_plan_set_fft_config applies a code (drops a cached graph).
+ * 1-D plans whose steps and rollouts run as one launch use the knobs in
+ * exmi_step_fourier, exmi_nonlinear and the derivatives only: that launch
+ * takes a fixed choice of radices, not reported here, until a code other than
+ * the reported one is set; giving the reported one back changes nothing.
  * (No reference counterpart: XLA picks the reference's FFT plans.) */
 int exmi_plan_fft_config(const exmi_plan* plan, int32_t* info, int32_t len);
 int exmi_plan_set_fft_config(exmi_plan* plan, int32_t code);

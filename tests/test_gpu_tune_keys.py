@@ -45,3 +45,29 @@ def test_each_is_timed_for_itself(device, pair, tmp_path, monkeypatch):
     keys = [ln.rsplit(" ", 1)[0] for ln in path.read_text().split("\n") if ln.strip()]
     # the old entry; a transform choice and a rollout strategy of each
     assert len(keys) == len(set(keys)) == 5, keys
+
+
+def test_the_reported_code_given_back_changes_nothing(device, tmp_path, monkeypatch):
+    """1-D plans step with radices of their own: reading a plan's knobs and
+    setting them again leaves every bit alone, another code is used there too."""
+    import torch
+
+    path = tmp_path / "tune.txt"
+    monkeypatch.setenv("EXMI_TUNE_CACHE", str(path))
+    make = lambda: S.Burgers(1, 1.0, 100, 1e-3, diffusivity=0.02)  # noqa: E731
+    make().fft_config(batch=3)
+    key = path.read_text().split("\n")[0].rsplit(" ", 1)[0]
+    path.write_text(f"{key} 101002048\n")  # two passes of ten points
+    st = make()
+    plan = st.plan(3)
+    cfg = plan.fft_config()
+    assert cfg["source"] == "cache" and cfg["radices"] == [10, 10]
+    plan.set_rollout_strategy(2)
+    u0 = torch.tensor(ics(3, 1, 1.0, 100, 5, seed=3)[0], device=device)
+    want = st.rollout_batch(u0, 8)
+    plan.set_fft_config(cfg["code"])
+    assert plan.fft_config()["code"] == cfg["code"]
+    assert torch.equal(st.rollout_batch(u0, 8), want)
+    plan.set_fft_config(200000 + 1024)  # 2 2 5 5
+    got = st.rollout_batch(u0, 8)
+    assert not torch.equal(got, want) and float((got - want).norm() / want.norm()) <= 3e-6
