@@ -62,18 +62,34 @@ def test_1d_one_launch_equals_separate_passes(device, N):
         assert torch.equal(st.repeat_batch(x, 3), tr[:, 3])
 
 
-def test_1d_per_member_tables_and_channels(device):
-    """Per-trajectory operators (lin_batch = B) and per-channel ones take
-    each workgroup's own tables."""
+@pytest.mark.parametrize("nt", [2, -1])
+def test_1d_per_member_tables_and_channels(device, nt):
+    """Per-trajectory operators (lin_batch = B) and per-channel ones take each
+    workgroup's own tables: a member's bits are those of its own plan with the
+    same strategy (the spectrum carried, or a float32 round trip per step:
+    other kernels, other bits), and the per-channel ones those of the oracle."""
     import torch
 
     nus = np.linspace(0.01, 0.05, 7)
-    ens = ex.ensemble(lambda nu: S.Burgers(1, 1.0, 77, 1e-3, diffusivity=float(nu)), nus)
-    u0 = torch.tensor(ics(7, 1, 1.0, 77, 5, seed=3)[0], device=device)
-    got = ens.rollout_batch(u0, 4)
-    for i, nu in enumerate(nus):
-        one = S.Burgers(1, 1.0, 77, 1e-3, diffusivity=float(nu)).rollout_batch(u0[i:i + 1], 4)
-        assert torch.equal(got[i:i + 1], one)
+    rates = [(2e-5, 1e-5), (4e-5, 1e-5), (3e-5, 2e-5)]
+    for name, make, ps, C in (("burgers", lambda nu: S.Burgers(1, 1.0, 77, 1e-3, diffusivity=float(nu)), nus, 1),
+                              ("gray-scott", lambda d: S.reaction.GrayScott(1, 2.5, 77, 1.0, diffusivity_1=d[0],
+                                                                            diffusivity_2=d[1]), rates, 2)):
+        print(f"[case] {name} strategy {nt}", flush=True)
+        B = len(ps)
+        ens = ex.ensemble(make, ps)
+        u0 = torch.tensor(0.5 * ics(B, 1, 1.0, 77, 5, seed=3, channels=C)[0], device=device)
+        ens.plan(B).set_rollout_strategy(nt)
+        got = ens.rollout_batch(u0, 4)
+        for i, v in enumerate(ps):
+            one = make(v)
+            one.plan(1).set_rollout_strategy(nt)
+            assert torch.equal(got[i:i + 1], one.rollout_batch(u0[i:i + 1], 4)), (name, i)
+    cpu = ost.GrayScott(1, 2.5, 77, 1.0, diffusivity_1=rates[1][0], diffusivity_2=rates[1][1], dtype=np.float32)
+    u = u0[1:2].cpu().numpy()
+    for s in range(4):
+        u = cpu.step_batch(u)
+        assert max_rel_l2(got[1:2, s].cpu().numpy(), u) <= RTOL_STEP
 
 
 @pytest.mark.parametrize("N", [6, 33, 99, 810, 825, 1025])
