@@ -2665,9 +2665,12 @@ static int effective_nt(const exmi_plan* p) {
     return p->fr2d ? 2 : -1;
   }
   // 1-D: the latency variant while it needs no more wavefronts than there are
-  // SIMDs (us per 100 KS steps, usual / latency, N = 256: 1024 trajectories
-  // 336 / 287, 2048 378 / 327, 4096 403 / 410, 8192 510 / 723)
-  if (p->roll[3] && (long long)p->d.batch * p->d.num_channels * (p->M / 4) <= 1024 * 64LL) return 3;
+  // SIMDs, the last whole number up to which no size loses much (us per 100 KS
+  // steps of repeat, one transform per lane group / two / latency variant, at 1
+  // and 2 wavefronts per SIMD: N = 64 204 / 327 / 215 and 228 / 369 / 280, 256
+  // 276 / 438 / 262 and 304 / 485 / 314, 512 300 / 472 / 260 and 312 / 499 / 309,
+  // 2048 583 / 1122 / 504 and 684 / 1175 / 597)
+  if (p->roll[3] && (long long)p->d.batch * p->d.num_channels * (p->M / latency_pt(p->M)) <= 1024 * 64LL) return 3;
   return p->roll[2] ? 2 : (p->roll[1] ? 1 : -1);
 }
 

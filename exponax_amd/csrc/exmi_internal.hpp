@@ -52,6 +52,18 @@ __host__ __device__ inline int num_coefs_c(int order, bool cplx) {
   return num_coefs(order) + (cplx ? (order >= 3 ? 2 : 1) : 0);
 }
 
+// Points per lane of the 1-D rollouts' latency variant (strategy 3) at M = N/2:
+// half the usual, twice the lanes per transform. With few trajectories a step
+// is one wavefront's serial chain of instruction issue, and half the points per
+// lane is about half the instructions, against one more LDS exchange per
+// transform. us per 100 KS steps, usual / latency variant: N = 64 243 / 186,
+// 128 264 / 194, 256 331 / 232, 512 348 / 237, 2048 716 / 572 for one
+// trajectory. Not at N = 1024 (M = 512), whose transform would leave its one
+// wavefront for two with a barrier per exchange (379 / 430). 0: not built.
+__host__ __device__ constexpr int latency_pt(int m) {
+  return m == 1024 ? 8 : (m >= 32 && m <= 256 && (m & (m - 1)) == 0) ? 4 : 0;
+}
+
 // Which states of a rollout of n steps are written: those after every,
 // 2 every, ... steps and the one after the last step (every = 1: all of them,
 // n: only the last). next_written: the step after which the next one is

@@ -153,17 +153,6 @@ static RollFn pick_roll_kc(int kind) {
   }
 }
 
-// Points per lane of the latency variant (nt = 3): half the usual, twice the
-// lanes per transform. With few trajectories a step is one wavefront's serial
-// chain of instruction issue, and half the points per lane is about half the
-// instructions, against one more LDS exchange per transform. us per 100 KS
-// steps, usual / latency variant: N = 64 243 / 186, 128 264 / 194, 256 331 /
-// 232, 512 348 / 237, 2048 716 / 572 for one trajectory; equal at 4096
-// trajectories of N = 64 to 256. Not at N = 1024 (M = 512), whose transform
-// would leave its one wavefront for two with a barrier per exchange (379 /
-// 430). 0: not built.
-constexpr int latency_pt(int m) { return m == 1024 ? 8 : (m >= 32 && m <= 256 && (m & (m - 1)) == 0) ? 4 : 0; }
-
 // Multi-step kernels carrying 1 or 2 transforms per lane group (nt = 1, 2),
 // or 1 on twice the lanes (nt = 3); `fr` selects the Fourier-resident variant
 // (ETDRK2 only); `std_kc` says that the plan's dealias cutoff is

@@ -63,3 +63,21 @@ def test_not_built_elsewhere(device):
                S.KortewegDeVries(1, 20.0, 256, 1e-3), S.reaction.AllenCahn(1, 1.0, 256, 1e-3)):
         with pytest.raises(NotImplementedError):
             st.plan(2).set_rollout_strategy(3)
+
+
+@pytest.mark.parametrize("N,B", [(64, 8192), (64, 8193), (256, 2048), (256, 2049), (2048, 512), (2048, 513)])
+def test_untuned_repeat_takes_it_up_to_one_wavefront_per_simd(device, N, B):
+    """A repeat before any rollout was timed: strategy 3 as long as its
+    wavefronts (two per transform at N = 2048) are no more than the 1024 SIMDs,
+    2 above. The strategies' bits tell which one ran."""
+    import torch
+
+    st = S.KuramotoSivashinskyConservative(1, 100.0 * N / 256, N, 0.05)
+    x = torch.tensor(ics(8, 1, 1.0, N, 5, seed=N)[0], device=device).repeat(B // 8 + 1, 1, 1)[:B].contiguous()
+    got = st.repeat_batch(x, 20)
+    bits = {}
+    for nt in (2, 3):
+        st.plan(B).set_rollout_strategy(nt)
+        bits[nt] = st.repeat_batch(x, 20)
+    assert not torch.equal(bits[2], bits[3])
+    assert torch.equal(got, bits[2 if B % 2 else 3])
