@@ -218,12 +218,16 @@ hipError_t launch_gprod(const GfftCfg& c, const NL3DArgs& a, const cf* F, cf* P,
   g.rows = a.dims == 3 ? (long long)a.nx * a.ny : a.ny;
   g.nunits = a.ninst / a.channels * ((g.rows + 1) / 2);
   g.units = c.lpb / most;  // the tuned lines per workgroup
-  // Short lines leave most of a workgroup's lanes without a butterfly: at
-  // least about 1152 points to a workgroup while that leaves three workgroups
-  // to a CU (3-D Burgers, two of 12 fields, two units instead of one: 20 steps
-  // at 48^3 2266 -> 2090 us, 16 at 45^3 1751 -> 1585; four vorticity fields of
-  // 16 x 135^2, 1088 units, would lose 1015 -> 1047).
-  long long fill = 1152 / ((long long)most * c.n);
+  // Short lines leave most of a workgroup's lanes without a butterfly: up to
+  // 1400 points to a workgroup while that leaves three workgroups to a CU (3-D
+  // Burgers, two of 12 fields, two units instead of one: 20 steps at 48^3 2266
+  // -> 2090 us, 16 at 45^3 1751 -> 1585; four vorticity fields of 16 x 135^2,
+  // 1088 units, would lose 1015 -> 1047). Swept from 0 to 3500 points over 21
+  // shapes, 16 steps (none / 1152 / 1400 / 1800 points): 3-D Burgers 2 x 48^3
+  // 1548 / 1430 / 1434 / 1465 us, 2 x 54^3 1830 / 1872 / 1731 / 1697,
+  // Navier-Stokes 4 x 50^3 1708 / 1634 / 1621 / 1671; the others of 1152 points
+  // and more within 1%.
+  long long fill = 1400 / ((long long)most * c.n);
   if (fill > g.nunits / 768) fill = g.nunits / 768;
   if (fill > GFFT_MAX_LINES / most) fill = GFFT_MAX_LINES / most;
   if (g.units < fill) g.units = (int)fill;
