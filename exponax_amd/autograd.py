@@ -4,8 +4,8 @@ whose backward passes run the hand-written adjoint kernels.
 The reference gets its derivatives from ``jax.grad`` through ``lax.scan``
 (``_utils.py:92-254``, README.md:85-91). It keeps every step's residuals. Here
 one state every ``checkpoint_every`` steps is kept (by the forward pass of
-``repeat``, by the backward of ``rollout``) and each segment is recomputed on
-the way back.
+``repeat`` where it passes them, else by the backward) and each segment is
+recomputed on the way back.
 
     u0 = torch.randn(32, 1, 128, 128, device="cuda", requires_grad=True)
     uT = exponax_amd.autograd.repeat(stepper, u0, 50, checkpoint_every=10)
@@ -93,9 +93,11 @@ def repeat(stepper, u0, n: int, *, checkpoint_every: int = 10):
     """``exponax.repeat(stepper, n)(u0)``, differentiable in ``u0``: the bits
     of ``stepper.repeat_batch``. Where a gradient can follow, the states after
     every ``checkpoint_every`` steps are kept with the graph until its backward
-    (ceil(n / checkpoint_every) - 1 batches of states)."""
+    (ceil(n / checkpoint_every) - 1 batches of states; in 1-D for the runtime
+    sizes only)."""
     _check(u0)
-    keep = torch.is_grad_enabled() and u0.requires_grad and _own_repeat(stepper) and 0 < (checkpoint_every or 0) < n
+    keep = (torch.is_grad_enabled() and u0.requires_grad and 0 < (checkpoint_every or 0) < n and _own_repeat(stepper)
+            and _writes_checkpoints(stepper, u0))
     return _Repeat.apply(u0, stepper, n, checkpoint_every, keep)
 
 
@@ -105,3 +107,12 @@ def _own_repeat(stepper):
     return (isinstance(stepper, BaseStepper) and getattr(stepper, "_groups", None) is None
             and type(stepper).repeat_batch in (BaseStepper.repeat_batch, Ensemble.repeat_batch)
             and type(stepper).rollout_vjp is BaseStepper.rollout_vjp)
+
+
+def _writes_checkpoints(stepper, u0):
+    """Whether the steps up to the end pass the checkpoints on their way: not
+    the one launch of the fused 1-D sizes, whose backward forms them as
+    ``rollout_vjp`` does."""
+    if stepper.num_spatial_dims > 1:
+        return True
+    return stepper.plan(stepper._split(u0, stepper.state_shape)[1]).fft_config() is not None

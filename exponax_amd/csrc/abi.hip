@@ -1337,10 +1337,10 @@ static hipError_t stages3d(exmi_plan* p, Stage3DArgs& sa, hipStream_t st, cf* em
   return e;
 }
 
-// The multi-step launches below write the states after every, 2 every, ...
-// steps and the last one (1: every state, n: the last one only) to out +
-// b * out_bs, one out_ts apart; the last one to last + b * out_bs instead
-// where that is given (next_written, written_at).
+// The multi-step launches below, those of the fused 1-D sizes apart, write the
+// states after every, 2 every, ... steps and the last one (1: every state, n:
+// the last one only) to out + b * out_bs, one out_ts apart; the last one to
+// last + b * out_bs instead where that is given (next_written, written_at).
 
 // 1-D plans of a runtime size that fit LDS (p->g1): n steps in one launch;
 // roundtrip: every step starts from the emitted float32 state, else the
@@ -2149,7 +2149,7 @@ int exmi_plan_get_tables(const exmi_plan* p, float* host_out, int64_t host_count
 }
 
 static int enqueue_roll(exmi_plan* p, int nt, const float* u0, long long u0_bs, float* out, long long out_bs,
-                        long long out_ts, int n, int every, float* last, hipStream_t st, int* first_bad = nullptr,
+                        long long out_ts, int n, int final_only, hipStream_t st, int* first_bad = nullptr,
                         float bound = 0.f, int bad_offset = 0);
 
 static int run_step(exmi_plan* p, const void* in, long long in_bs, int in_f, void* out, long long out_bs, int out_f,
@@ -2167,7 +2167,7 @@ static int run_step(exmi_plan* p, const void* in, long long in_bs, int in_f, voi
     if (nonlin_only || in_f || out_f)
       return fail(EXMI_ERR_UNSUPPORTED, "channel-coupled reaction plans step physical states only");
     const long long sz = (long long)p->d.num_channels * p->d.num_points;
-    return enqueue_roll(p, 1, (const float*)in, in_bs, (float*)out, out_bs, sz, 1, 1, nullptr, st);
+    return enqueue_roll(p, 1, (const float*)in, in_bs, (float*)out, out_bs, sz, 1, 0, st);
   }
   hipError_t e = nonlin_only ? p->nonlin(a, st) : p->step(a, st);
   if (e != hipSuccess) return fail(EXMI_ERR_HIP, "step launch failed: %s", hipGetErrorString(e));
@@ -2233,7 +2233,7 @@ static hipError_t copy_batch(const float* src, long long ss, float* dst, long lo
 }
 
 static int enqueue_roll(exmi_plan* p, int nt, const float* u0, long long u0_bs, float* out, long long out_bs,
-                        long long out_ts, int n, int every, float* last, hipStream_t st, int* first_bad,
+                        long long out_ts, int n, int final_only, hipStream_t st, int* first_bad,
                         float bound, int bad_offset) {
   Roll1DArgs ra;
   fill_args(p, &ra.s);
@@ -2246,8 +2246,7 @@ static int enqueue_roll(exmi_plan* p, int nt, const float* u0, long long u0_bs, 
   ra.traj_bstride = out_bs;
   ra.traj_tstride = out_ts;
   ra.nsteps = n;
-  ra.every = every;
-  ra.last = last;
+  ra.final_only = final_only;
   hipError_t e = p->roll[nt](ra, st);
   return e == hipSuccess ? EXMI_OK : fail(EXMI_ERR_HIP, "rollout launch failed: %s", hipGetErrorString(e));
 }
@@ -2367,7 +2366,7 @@ static int enqueue_rollout_nt(exmi_plan* p, int nt, const float* u0, long long u
   // nt = -1 on a plan that chose the Fourier-resident kernels itself: the
   // per-step launches (the literal physical round trip) stay available
   if (p->fourier_resident && (nt == 0 || (nt < 0 && !p->fr_auto))) nt = p->roll[2] ? 2 : 1;
-  if (nt > 0 && p->roll[nt]) return enqueue_roll(p, nt, u0, u0_bs, traj + off * sz, tstride, sz, n, 1, nullptr, st);
+  if (nt > 0 && p->roll[nt]) return enqueue_roll(p, nt, u0, u0_bs, traj + off * sz, tstride, sz, n, 0, st);
   for (int t = 0; t < n; ++t) {
     const float* in = (t == 0 && !include_init) ? u0 : traj + (long long)(t - 1 + off) * sz;
     const long long ibs = (t == 0 && !include_init) ? u0_bs : tstride;
@@ -2678,10 +2677,9 @@ static int effective_nt(const exmi_plan* p) {
 // one segment).
 static int vjp_segment(int n, int every) { return every > 0 && every < n ? every : (n > 0 ? n : 1); }
 
-// n steps from u0 (batch stride s) to out, whose states after K, 2 K, ... < n
-// steps also go to ckpt (none with K >= n), each a contiguous batch: of every
-// strategy the rollout whose last state alone is written without them, so the
-// result does not depend on K.
+// n steps from u0 (batch stride s) to out; the states after K, 2 K, ... < n
+// steps also go to ckpt (none with K >= n), each a contiguous batch. out is the
+// last state of the rollout that writes it alone, whatever K.
 static int enqueue_repeat(exmi_plan* p, const float* u0, long long s, float* out, int n, int K, float* ckpt,
                           hipStream_t st) {
   const long long sz = state_size(p), bsz = (long long)p->d.batch * sz;
@@ -2718,7 +2716,18 @@ static int enqueue_repeat(exmi_plan* p, const float* u0, long long s, float* out
     return EXMI_OK;
   }
   const int nt = effective_nt(p);
-  if (nt > 0 && p->roll[nt]) return enqueue_roll(p, nt, u0, s, first, sz, bsz, n, K, last, st);
+  if (nt > 0 && p->roll[nt]) {
+    // these kernels write every state or the last one only (a third way of
+    // writing costs them registers, and at N = 2048 a wavefront per SIMD: 365 ->
+    // 679 us of 50 KS steps of 1500 trajectories), so the checkpoints are formed
+    // by segments of their own
+    int rc = EXMI_OK;
+    for (int t = K; t < n && !rc; t += K) {
+      float* c = ckpt + (long long)(t / K - 1) * bsz;
+      rc = enqueue_roll(p, nt, t == K ? u0 : c - bsz, t == K ? s : sz, c, sz, 0, K, 1, st);
+    }
+    return rc ? rc : enqueue_roll(p, nt, u0, s, out, sz, 0, n, 1, st);
+  }
   const float* in = u0;
   for (int t = 0; t < n; ++t) {  // in turn to out and the workspace, the last one to out
     float* o = state(t);
@@ -2808,7 +2817,7 @@ int exmi_rollout_checked(exmi_plan* p, const float* u0, int64_t u0_bs, float* tr
     }
     hipLaunchKernelGGL(exmi_fill_int_kernel, dim3(small_grid(B)), dim3(256), 0, st, (int*)first_bad, B, INT_MAX);
     HIP_TRY(hipGetLastError());
-    int rc = enqueue_roll(p, nt, u0, u0_bs, traj + off * sz, tstride, sz, n, 1, nullptr, st, (int*)first_bad, bnd, off);
+    int rc = enqueue_roll(p, nt, u0, u0_bs, traj + off * sz, tstride, sz, n, 0, st, (int*)first_bad, bnd, off);
     if (rc) return rc;
     hipLaunchKernelGGL(exmi_bad_finalize_kernel, dim3(small_grid(B)), dim3(256), 0, st, (int*)first_bad, B);
     HIP_TRY(hipGetLastError());

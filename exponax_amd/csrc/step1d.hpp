@@ -763,32 +763,35 @@ inline hipError_t launch_step1d(const Step1DArgs& a, hipStream_t st) {
 // operator tables and twiddles on chip for `nsteps` steps. Per step the
 // arithmetic is exactly that of step1d_kernel (physical state in float32 ->
 // forward transform -> ETDRK step -> inverse transform -> float32 state);
-// the states named by `every` are written. Every wave runs the same bounded
-// loop; there is no inter-wave communication.
+// the new state is written to traj[b, t0 + step] (or only the final state
+// when `final_only`). Every wave runs the same bounded loop; there is no
+// inter-wave communication.
 struct Roll1DArgs {
   Step1DArgs s;            // in, in_bstride: initial states (physical)
   float* traj;             // output base
   long long traj_bstride;  // floats between trajectories
   long long traj_tstride;  // floats between consecutive outputs of one trajectory
   int nsteps;
-  int every;               // written: the states after every, 2 every, ... steps and the last one
-  float* last = nullptr;   // where the last one goes, or null: in its turn
+  int final_only;          // 1: write only the last state (traj_tstride unused)
   int* first_bad = nullptr;  // failure detection, or nullptr: per trajectory, atomicMin of the first
-                             // written slot (bad_offset + its number) holding a value that is not finite or
+                             // written slot (bad_offset + step) holding a value that is not finite or
                              // exceeds `bound` in magnitude
   float bound = 0.f;
   int bad_offset = 0;
 };
 
-// Write the NT physical states (N x, times `scale`) of a step to `to`.
+// Write the NT physical states (N x, times `scale`) of a step to the
+// trajectory buffer.
 template <int M, int PT, int NT>
 __device__ __forceinline__ void store_states(const cf (*S)[PT], float scale, const Roll1DArgs& ra, const int* tb_,
-                                             const int* cb_, const bool* act, float* to, int j) {
+                                             const int* cb_, const bool* act, int step, int j) {
   constexpr int T = M / PT;
+  const long long tofs = ra.final_only ? 0 : (long long)step * ra.traj_tstride;
 #pragma unroll
   for (int n = 0; n < NT; ++n) {
     if (act[n]) {
-      float2* out = reinterpret_cast<float2*>(to + (long long)tb_[n] * ra.traj_bstride + (long long)cb_[n] * 2 * M);
+      float2* out = reinterpret_cast<float2*>(ra.traj + (long long)tb_[n] * ra.traj_bstride + tofs +
+                                              (long long)cb_[n] * 2 * M);
 #pragma unroll
       for (int s = 0; s < PT; ++s) out[j + s * T] = make_float2(S[n][s].re * scale, S[n][s].im * scale);
     }
@@ -869,12 +872,12 @@ __global__ void __launch_bounds__((M / PT) > 64 ? (M / PT) : 64) roll1d_kernel(R
     }
   }
 
-  // failure detection: the first slot whose written state fails the bound
+  // failure detection: the first step whose written state fails the bound
   // (a lane's own values; the trajectory's minimum is taken at the end)
   int fb[NT];
 #pragma unroll
   for (int n = 0; n < NT; ++n) fb[n] = INT_MAX;
-  auto check = [&](const cf (*V)[PT], float scale, int slot) {
+  auto check = [&](const cf (*V)[PT], float scale, int step) {
     if (!ra.first_bad) return;
 #pragma unroll
     for (int n = 0; n < NT; ++n) {
@@ -882,18 +885,16 @@ __global__ void __launch_bounds__((M / PT) > 64 ? (M / PT) : 64) roll1d_kernel(R
 #pragma unroll
       for (int s = 0; s < PT; ++s)
         bad |= !(fabsf(V[n][s].re * scale) <= ra.bound) | !(fabsf(V[n][s].im * scale) <= ra.bound);
-      if (bad && fb[n] == INT_MAX) fb[n] = slot;
+      if (bad && fb[n] == INT_MAX) fb[n] = step;
     }
   };
 
   if constexpr (FR) rfft_l<LAY, M, PT, NT>(S, nyq, ln, lds, rt);
-  int slot = 0, next = next_written(0, ra.every, ra.nsteps);
   for (int step = 0; step < ra.nsteps; ++step) {
     if constexpr (!FR) rfft_l<LAY, M, PT, NT>(S, nyq, ln, lds, rt);
     if constexpr (FOLD) etdrk2_folded<KIND, M, PT, NT, KC>(FR ? 1.f : 1.f / (r2n * r2n), S, nyq, cl, ln, lds, rt, a.kscale);
     else etdrk_step<KIND, ORDER, M, PT, NT, CL, LAY, CPLX>(S, nyq, cl, ln, lds, rt, a);
-    const bool emit = step + 1 == next;
-    float* const to = written_at(ra.traj, ra.traj_tstride, slot, ra.last, step + 1 == ra.nsteps);
+    const bool emit = !ra.final_only || step == ra.nsteps - 1;
     if constexpr (FR) {
       if (emit) {
         cf O[NT][PT];
@@ -905,8 +906,8 @@ __global__ void __launch_bounds__((M / PT) > 64 ? (M / PT) : 64) roll1d_kernel(R
           for (int s = 0; s < PT; ++s) O[n][s] = S[n][s];
         }
         irfft_l<LAY, M, PT, NT>(O, on, ln, lds, rt);
-        store_states<M, PT, NT>(O, r2n, ra, tb_, cb_, act, to, j);
-        check(O, r2n, slot);
+        store_states<M, PT, NT>(O, r2n, ra, tb_, cb_, act, step, j);
+        check(O, r2n, step);
       }
     } else {
       irfft_l<LAY, M, PT, NT>(S, nyq, ln, lds, rt);
@@ -920,19 +921,15 @@ __global__ void __launch_bounds__((M / PT) > 64 ? (M / PT) : 64) roll1d_kernel(R
           for (int s = 0; s < PT; ++s) S[n][s] = cf{S[n][s].re * r2n, S[n][s].im * r2n};
       }
       if (emit) {
-        store_states<M, PT, NT>(S, 1.f, ra, tb_, cb_, act, to, j);
-        check(S, 1.f, slot);
+        store_states<M, PT, NT>(S, 1.f, ra, tb_, cb_, act, step, j);
+        check(S, 1.f, step);
       }
-    }
-    if (emit) {
-      ++slot;
-      next = next_written(next, ra.every, ra.nsteps);
     }
   }
   if (ra.first_bad) {
 #pragma unroll
     for (int n = 0; n < NT; ++n)
-      if (act[n] && fb[n] != INT_MAX) atomicMin(ra.first_bad + tb_[n], ra.bad_offset + fb[n]);
+      if (act[n] && fb[n] != INT_MAX) atomicMin(ra.first_bad + tb_[n], ra.bad_offset + (ra.final_only ? 0 : fb[n]));
   }
 }
 

@@ -52,8 +52,12 @@ def test_kept_checkpoints_give_the_gradient(device, name, n, every):
         out, ckpt = st._repeat_checkpointed(u0, n, every)
         assert torch.equal(out, ref), nt
         assert ckpt.shape[0] == -(-n // K) - 1
-        if nt != 0:  # (a rollout with 0 would choose a strategy)
-            assert torch.equal(ckpt, st.rollout_batch(u0, n)[:, K - 1:n - 1:K].movedim(1, 0)), nt
+        if nt != 0 and len(ckpt):  # (a rollout with 0 would choose a strategy)
+            states = st.rollout_batch(u0, n)[:, K - 1:n - 1:K].movedim(1, 0)
+            if name == "ks1d_128":  # formed by segments of their own
+                assert float((ckpt - states).norm() / states.norm()) <= 1e-6, nt
+            else:
+                assert torch.equal(ckpt, states), nt
         want = st.rollout_vjp(u0, n, g_final=g, checkpoint_every=every)
         for v in (u0, wide):
             x = v.detach().requires_grad_(True)
@@ -70,8 +74,8 @@ def test_only_a_graph_keeps_checkpoints(device, monkeypatch):
     for one."""
     import torch
 
-    st = S.KuramotoSivashinskyConservative(1, 30.0, 64, 0.05)
-    x = torch.tensor(ics(2, 1, 1.0, 64, 3, seed=5)[0], device=device, requires_grad=True)
+    st = S.KuramotoSivashinskyConservative(1, 30.0, 60, 0.05)
+    x = torch.tensor(ics(2, 1, 1.0, 60, 3, seed=5)[0], device=device, requires_grad=True)
     ref = st.repeat_batch(x.detach(), 6)
     kept = []
     monkeypatch.setattr(type(st), "_repeat_checkpointed",
@@ -81,7 +85,12 @@ def test_only_a_graph_keeps_checkpoints(device, monkeypatch):
     assert torch.equal(ex.autograd.repeat(st, x.detach(), 6, checkpoint_every=2), ref)
     assert not kept
     ex.autograd.repeat(st, x, 6, checkpoint_every=2)
-    assert kept
+    assert kept == [1]
+    # the fused 1-D sizes pass no checkpoints on their way
+    fused = S.KuramotoSivashinskyConservative(1, 30.0, 64, 0.05)
+    y = torch.tensor(ics(2, 1, 1.0, 64, 3, seed=5)[0], device=device, requires_grad=True)
+    assert torch.equal(ex.autograd.repeat(fused, y, 6, checkpoint_every=2), fused.repeat_batch(y.detach(), 6))
+    assert kept == [1]
 
 
 def test_a_steppers_own_repeat_is_called(device):
@@ -96,12 +105,12 @@ def test_a_steppers_own_repeat_is_called(device):
         def rollout_vjp(self, *a, **kw):
             return 2.0 * super().rollout_vjp(*a, **kw)
 
-    u0 = torch.tensor(ics(2, 1, 1.0, 64, 3, seed=5)[0], device=device)
-    plain = S.KuramotoSivashinskyConservative(1, 30.0, 64, 0.05)
+    u0 = torch.tensor(ics(2, 1, 1.0, 60, 3, seed=5)[0], device=device)
+    plain = S.KuramotoSivashinskyConservative(1, 30.0, 60, 0.05)
     x = u0.clone().requires_grad_(True)
-    assert torch.equal(ex.autograd.repeat(Mine(1, 30.0, 64, 0.05), x, 6, checkpoint_every=2),
+    assert torch.equal(ex.autograd.repeat(Mine(1, 30.0, 60, 0.05), x, 6, checkpoint_every=2),
                        2.0 * plain.repeat_batch(u0, 6))
-    (got,) = torch.autograd.grad(ex.autograd.repeat(Scaled(1, 30.0, 64, 0.05), x, 6, checkpoint_every=2).sum(), x)
+    (got,) = torch.autograd.grad(ex.autograd.repeat(Scaled(1, 30.0, 60, 0.05), x, 6, checkpoint_every=2).sum(), x)
     want = 2.0 * plain.rollout_vjp(u0, 6, g_final=torch.ones_like(u0), checkpoint_every=2)
     assert torch.equal(got, want)
 
@@ -111,8 +120,8 @@ def test_saved_tensor_hooks(device):
     comes back is looked at before a kernel reads it."""
     import torch
 
-    st = S.KuramotoSivashinskyConservative(1, 30.0, 64, 0.05)
-    x = torch.tensor(ics(2, 1, 1.0, 64, 3, seed=5)[0], device=device, requires_grad=True)
+    st = S.KuramotoSivashinskyConservative(1, 30.0, 60, 0.05)
+    x = torch.tensor(ics(2, 1, 1.0, 60, 3, seed=5)[0], device=device, requires_grad=True)
     y = ex.autograd.repeat(st, x, 6, checkpoint_every=2)
     (want,) = torch.autograd.grad(y.sum(), x)
     hooks = {"cpu": (lambda t: t.cpu(), lambda t: t),
