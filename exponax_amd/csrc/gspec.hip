@@ -2,13 +2,14 @@
 // set) around the line transforms of gfft.hpp: the spectral fields with the
 // first inverse axis, the rows of the last axis with the pointwise products,
 // and in 1-D whole ETDRK rollouts in one launch.
-// One nonlinear evaluation of eight 513^2 Kolmogorov instances: 28 us of
-// fields, 46 us of rows and products, 25 us of forward lines with the stage,
+// One nonlinear evaluation of eight 513^2 Kolmogorov instances: 27 us of
+// fields, 41 us of rows and products, 24 us of forward lines with the stage,
 // against 358 us as separate fields, transforms of whole fields (119 + 88 us
 // for the four fields), products, transforms and stage. What bounds them is
 // the latency of the short passes between barriers at three to five
 // workgroups per CU; passes in place in registers (half the LDS, twice the
-// barriers) gave 42 us for the rows at 513 and cost 8% of a step at 48^3.
+// barriers) took the rows at 513 from 48 to 42 us when the odd sizes' lines
+// still had a pad entry per point, and cost 8% of a step at 48^3.
 #include "gspec.hpp"
 #include "nl3d.hpp"
 

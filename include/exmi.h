@@ -289,7 +289,9 @@ int exmi_rollout_vjp(exmi_plan* plan, const float* u0, int64_t u0_bstride, int32
  * (ceil(n/K) - 1, B, C, N^D) contiguous, the caller's to hold until the
  * gradient is taken. exmi_repeat_vjp with the same n_steps, checkpoint_every
  * and ckpt is exmi_rollout_vjp(..., g_final, ...) without its forward pass.
- * ckpt may be NULL where it holds nothing. Not captured into a graph. */
+ * ckpt may be NULL where it holds nothing. Not captured into a graph. On the
+ * fused 1-D sizes the kept states take launches of their own, so nothing is
+ * saved there. */
 int exmi_repeat_checkpointed(exmi_plan* plan, const float* u0, int64_t u0_bstride, float* u_out, float* ckpt,
                              int32_t n_steps, int32_t checkpoint_every, void* stream);
 int exmi_repeat_vjp(exmi_plan* plan, const float* u0, int64_t u0_bstride, int32_t n_steps, const float* ckpt,
@@ -426,8 +428,9 @@ int exmi_cnn_forward(const float* params, int32_t num_points, int32_t count, con
 /* Gradients of sum(y * dy) for the samples of the last exmi_cnn_forward into
  * `workspace`: dparams (EXMI_CNN_NUM_PARAMS, overwritten, summed over the
  * samples) and, when dx is not NULL, dx (count, num_points). The weight
- * gradients are reduced over per-wavefront partial sums in a fixed order
- * (deterministic). */
+ * gradients are reduced over per-workgroup partial sums in a fixed order
+ * (deterministic). The partial sums and the layers' deltas are written into
+ * the workspace, so two calls on one workspace must not overlap. */
 int exmi_cnn_backward(const float* params, int32_t num_points, int32_t count, const float* dy, float* dx,
                       float* dparams, void* workspace, void* stream);
 
